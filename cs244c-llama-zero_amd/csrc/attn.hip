@@ -20,15 +20,10 @@
 // group and the query blocks at or after the diagonal) and a dQ pass (one
 // workgroup per 128 queries, looping over key blocks up to the diagonal); no
 // atomics, deterministic.
-#include "lz_common.h"
+#include "attn_tiles.h"
+#include "attn_wave.h"
 
 namespace {
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kLn2 = 0.6931471805599453f;
 
 struct AttnArgs {
   const uint16_t* q;
@@ -38,13 +33,9 @@ struct AttnArgs {
   uint16_t* o;
   int64_t ldo;
   float* lse;
-  const uint16_t* vt;  // fwd: V^T [B,KV,hd,S]
   // backward
-  const uint16_t* qt;   // [B,H,hd,S]
-  const uint16_t* kt;   // [B,KV,hd,S]
   const uint16_t* dout; // rows like o
   int64_t lddo;
-  const uint16_t* dot;  // dO^T [B,H,hd,S]
   const float* delta;   // [B,H,S] rowsum(dO*O)
   float* delta_w;       // the same rows, written by the dQ kernel that computes them (with o as O)
   uint16_t* dq;
@@ -58,112 +49,6 @@ struct AttnArgs {
   int B, S, H, KV;
   float scale;
 };
-
-// Workgroup -> (query block, batch, head), heaviest query blocks first.  The
-// hardware deals workgroup i to XCD i % 8; when the (batch, kv head) pairs
-// split evenly over the 8 XCDs, each XCD gets its own pairs, and all query
-// heads of a pair's group and neighbouring query blocks run on that XCD at
-// about the same time, so the K and V rows they stream are fetched into its
-// L2 once instead of by workgroups spread over every XCD.
-__device__ __forceinline__ void query_block_coords(int bid, int nqb, int B, int H, int KV, int& qb, int& b, int& h) {
-  const int rep = H / KV, npairs = B * KV;
-  if (npairs % 8 == 0) {
-    const int xcd = bid % 8, j = bid / 8;
-    const int per_q = (npairs / 8) * rep;  // workgroups of one query block on one XCD
-    const int qr = j / per_q, rem = j - qr * per_q;
-    const int pair = xcd + 8 * (rem / rep);
-    b = pair / KV;
-    h = (pair % KV) * rep + rem % rep;
-    qb = nqb - 1 - qr;
-  } else {
-    const int bh = B * H;
-    qb = nqb - 1 - bid / bh;
-    b = (bid % bh) / H;
-    h = bid % H;
-  }
-}
-
-// Workgroup -> (key block, batch, kv head), first key blocks (the most
-// queries at or after them) first; pairs split over XCDs as above, so the Q
-// and dO rows a pair's key blocks read share an L2.
-__device__ __forceinline__ void key_block_coords(int bid, int B, int KV, int& kvb, int& b, int& g) {
-  const int npairs = B * KV;
-  int pair;
-  if (npairs % 8 == 0) {
-    const int xcd = bid % 8, j = bid / 8, ppx = npairs / 8;
-    kvb = j / ppx;
-    pair = xcd + 8 * (j - kvb * ppx);
-  } else {
-    kvb = bid / npairs;
-    pair = bid % npairs;
-  }
-  b = pair / KV;
-  g = pair % KV;
-}
-
-// Elements e0..e0+7 of an accumulator -> an 8-element MFMA operand of the
-// 16-bit format F (fragments travel as bf16x8_t: 16 raw bytes per lane).
-template <typename F = FmtBF16>
-__device__ __forceinline__ bf16x8_t pack8(const f32x16_t& v, int e0) {
-  const uint4 w = make_uint4(F::pack2(v[e0], v[e0 + 1]), F::pack2(v[e0 + 2], v[e0 + 3]),
-                             F::pack2(v[e0 + 4], v[e0 + 5]), F::pack2(v[e0 + 6], v[e0 + 7]));
-  return __builtin_bit_cast(bf16x8_t, w);
-}
-
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-
-// One 32x32x16 MFMA on operands of the format F.
-template <typename F>
-__device__ __forceinline__ f32x16_t mfma16(const bf16x8_t& a, const bf16x8_t& b, const f32x16_t& c) {
-  if constexpr (F::kDtype == LZ_F16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c,
-                                                 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-
-// x combined with the value of lane ^ 32 (both halves get the same result):
-// v_permlane32_swap exchanges the halves of two registers without an LDS
-// round trip.
-__device__ __forceinline__ float max_halves(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float sum_halves(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-__device__ __forceinline__ bf16x8_t lds_frag16(const char* p) {
-  return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(p));
-}
-
-// Two 4-element runs (8 bytes each) -> one 8-element fragment.
-__device__ __forceinline__ bf16x8_t lds_frag_2x4(const char* p0, const char* p1) {
-  const uint2 a = *reinterpret_cast<const uint2*>(p0);
-  const uint2 b = *reinterpret_cast<const uint2*>(p1);
-  return __builtin_bit_cast(bf16x8_t, make_uint4(a.x, a.y, b.x, b.y));
-}
-
-// 8 consecutive elements of a row of length `len` starting at `idx` (multiple
-// of 8), zero outside [0, len).
-__device__ __forceinline__ uint4 load8(const uint16_t* row, int64_t idx, int64_t len) {
-  if (idx + 8 <= len && ((reinterpret_cast<uintptr_t>(row + idx) & 15) == 0))
-    return *reinterpret_cast<const uint4*>(row + idx);
-  uint16_t t[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) t[e] = (idx + e < len) ? row[idx + e] : (uint16_t)0;
-  return make_uint4((uint32_t)t[0] | ((uint32_t)t[1] << 16), (uint32_t)t[2] | ((uint32_t)t[3] << 16),
-                    (uint32_t)t[4] | ((uint32_t)t[5] << 16), (uint32_t)t[6] | ((uint32_t)t[7] << 16));
-}
-
-template <typename F = FmtBF16>
-__device__ __forceinline__ void store_bf16x4(uint16_t* p, float a, float b, float c, float d) {
-  uint2 w;
-  w.x = (uint32_t)F::from_f(a) | ((uint32_t)F::from_f(b) << 16);
-  w.y = (uint32_t)F::from_f(c) | ((uint32_t)F::from_f(d) << 16);
-  *reinterpret_cast<uint2*>(p) = w;
-}
 
 // One lane's row of a dQ or dK accumulator set (columns 32*i + 8*q4 +
 // 4*half + e, the MFMA output layout), times `scale`, stored as bf16 at dst.
@@ -226,442 +111,8 @@ __device__ __forceinline__ void store_grad_row(uint16_t* dst, const f32x16_t (&a
     }
 }
 
-// Row tile [rows][HD] (row stride `rb` bytes) from a [S, ld] row-major source.
-template <int HD, int ROWS, int NT>
-__device__ __forceinline__ void load_rows(char* dst, int rb, const uint16_t* src, int64_t ld, int64_t r0, int64_t nrows,
-                                          int tid) {
-  constexpr int kChunks = ROWS * HD / 8;
-#pragma unroll
-  for (int i = 0; i < (kChunks + NT - 1) / NT; ++i) {
-    const int c = tid + i * NT;
-    if (c < kChunks) {
-      const int row = c / (HD / 8), ch = c % (HD / 8);
-      const int64_t r = r0 + row;
-      uint4 val = make_uint4(0, 0, 0, 0);
-      if (r < nrows) val = *reinterpret_cast<const uint4*>(src + r * ld + ch * 8);
-      *reinterpret_cast<uint4*>(dst + row * rb + ch * 16) = val;
-    }
-  }
-}
-
-// Transposed tile [HD][COLS] (row stride `rb` bytes, a multiple of 8) from a
-// [HD, S] source, columns c0.. (zero beyond S).
-template <int HD, int COLS, int NT>
-__device__ __forceinline__ void load_trows(char* dst, int rb, const uint16_t* src, int64_t S, int64_t c0, int tid) {
-  constexpr int kChunks = HD * COLS / 8;
-#pragma unroll
-  for (int i = 0; i < (kChunks + NT - 1) / NT; ++i) {
-    const int c = tid + i * NT;
-    if (c < kChunks) {
-      const int row = c / (COLS / 8), ch = c % (COLS / 8);
-      const uint4 val = load8(src + (int64_t)row * S, c0 + ch * 8, S);
-      uint2* d = reinterpret_cast<uint2*>(dst + row * rb + ch * 16);
-      d[0] = make_uint2(val.x, val.y);
-      d[1] = make_uint2(val.z, val.w);
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// Forward.  256 threads; 128 queries per workgroup (32 per wave); 64-key
-// steps.  The K and V^T tiles of step i+1 are loaded into registers while step
-// i computes from the other LDS buffer, so global latency overlaps the MFMAs.
-// Softmax in log2 space: p = exp2(s*c - m) with c = scale*log2(e) folded into
-// one FMA; O and l are rescaled only when some lane's running max moved.
-// ---------------------------------------------------------------------------
-template <int HD>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) attn_fwd_kernel(AttnArgs a) {
-  constexpr int BQ = 128, BKV = 64, NT = 256;
-  constexpr int KROW = HD * 2 + 16;
-  constexpr int VROW = BKV * 2 + 8;
-  constexpr int kBuf = BKV * KROW + HD * VROW;
-  constexpr int kKC = BKV * HD / 8 / NT;  // 16-byte K chunks per thread per step
-  constexpr int kVC = HD * BKV / 8 / NT;  // 16-byte V^T chunks per thread per step
-  static_assert(kKC * NT * 8 == BKV * HD && kVC * NT * 8 == HD * BKV, "tile/thread mismatch");
-  __shared__ __attribute__((aligned(16))) char smem[2 * kBuf];
-
-  const int S = a.S, H = a.H, KV = a.KV;
-  const int nqb = (S + BQ - 1) / BQ;
-  int qb, b, h;
-  query_block_coords(blockIdx.x, nqb, a.B, H, KV, qb, b, h);
-  const int g = h / (H / KV);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int half = lane >> 5, l32 = lane & 31;
-  const int q0 = qb * BQ, qw0 = q0 + 32 * wave;
-  const int qrow = qw0 + l32;
-
-  bf16x8_t qf[HD / 16];
-  {
-    const uint16_t* qp = a.q + ((int64_t)b * S + min(qrow, S - 1)) * a.ldq + (int64_t)h * HD + 8 * half;
-#pragma unroll
-    for (int kk = 0; kk < HD / 16; ++kk) qf[kk] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(qp + kk * 16));
-  }
-  f32x16_t o[HD / 32];
-#pragma unroll
-  for (int i = 0; i < HD / 32; ++i)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
-  float m = -INFINITY, l = 0.f;
-  const float c = a.scale * kLog2e;
-
-  const int kv_end = min(S, q0 + BQ);
-  const int kv_end_w = min(S, qw0 + 32);
-  const uint16_t* kbase = a.k + (int64_t)b * S * a.ldk + (int64_t)g * HD;
-  const uint16_t* vtbase = a.vt + (int64_t)(b * KV + g) * HD * S;
-
-  uint4 kreg[kKC], vreg[kVC];
-  auto gload = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < kKC; ++i) {
-      const int cidx = tid + i * NT, row = cidx / (HD / 8), ch = cidx % (HD / 8);
-      const int r = k0 + row;
-      const uint4 v = *reinterpret_cast<const uint4*>(kbase + (int64_t)min(r, S - 1) * a.ldk + ch * 8);
-      const uint32_t msk = r < S ? ~0u : 0u;
-      kreg[i] = make_uint4(v.x & msk, v.y & msk, v.z & msk, v.w & msk);
-    }
-#pragma unroll
-    for (int i = 0; i < kVC; ++i) {
-      const int cidx = tid + i * NT, row = cidx / (BKV / 8), ch = cidx % (BKV / 8);
-      vreg[i] = load8(vtbase + (int64_t)row * S, k0 + ch * 8, S);
-    }
-  };
-  auto lstore = [&](char* buf) {
-#pragma unroll
-    for (int i = 0; i < kKC; ++i) {
-      const int cidx = tid + i * NT, row = cidx / (HD / 8), ch = cidx % (HD / 8);
-      *reinterpret_cast<uint4*>(buf + row * KROW + ch * 16) = kreg[i];
-    }
-#pragma unroll
-    for (int i = 0; i < kVC; ++i) {
-      const int cidx = tid + i * NT, row = cidx / (BKV / 8), ch = cidx % (BKV / 8);
-      uint2* d = reinterpret_cast<uint2*>(buf + BKV * KROW + row * VROW + ch * 16);
-      d[0] = make_uint2(vreg[i].x, vreg[i].y);
-      d[1] = make_uint2(vreg[i].z, vreg[i].w);
-    }
-  };
-
-  const int nsteps = (kv_end + BKV - 1) / BKV;
-  gload(0);
-  lstore(smem);
-  __syncthreads();
-  for (int it = 0; it < nsteps; ++it) {
-    const int k0 = it * BKV;
-    if (it + 1 < nsteps) gload(k0 + BKV);
-    const char* Ks = smem + (it & 1) * kBuf;
-    const char* Vts = Ks + BKV * KROW;
-    if (k0 < kv_end_w) {
-      f32x16_t s[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[t][r] = 0.f;
-#pragma unroll
-        for (int kk = 0; kk < HD / 16; ++kk) {
-          const bf16x8_t af = lds_frag16(Ks + (t * 32 + l32) * KROW + kk * 32 + half * 16);
-          s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, qf[kk], s[t], 0, 0, 0);
-        }
-      }
-      const bool need_mask = (k0 + BKV - 1 > qw0) || (k0 + BKV > S);
-      float mx = -INFINITY;
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          if (need_mask) {
-            const int kv = k0 + t * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-            if (kv > qrow || kv >= S) s[t][r] = -INFINITY;
-          }
-          mx = fmaxf(mx, s[t][r]);
-        }
-      mx = max_halves(mx);
-      const float m_new = fmaxf(m, mx * c);
-      const float nm = -m_new;
-      float rs = 0.f;
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float p = __builtin_amdgcn_exp2f(fmaf(s[t][r], c, nm));
-          s[t][r] = p;
-          rs += p;
-        }
-      rs = sum_halves(rs);
-      if (__builtin_amdgcn_read_exec() & __ballot(m_new != m)) {  // some lane's max moved
-        const float alpha = __builtin_amdgcn_exp2f(m - m_new);
-        l *= alpha;
-#pragma unroll
-        for (int i = 0; i < HD / 32; ++i)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
-      }
-      l += rs;
-      m = m_new;
-#pragma unroll
-      for (int ks = 0; ks < BKV / 16; ++ks) {
-        const bf16x8_t pb = pack8(s[ks >> 1], 8 * (ks & 1));
-#pragma unroll
-        for (int i = 0; i < HD / 32; ++i) {
-          const char* row = Vts + (i * 32 + l32) * VROW;
-          const bf16x8_t av = lds_frag_2x4(row + (16 * ks + 4 * half) * 2, row + (16 * ks + 8 + 4 * half) * 2);
-          o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, pb, o[i], 0, 0, 0);
-        }
-      }
-    }
-    if (it + 1 < nsteps) lstore(smem + ((it + 1) & 1) * kBuf);
-    __syncthreads();
-  }
-  if (qrow < S) {
-    const float inv_l = 1.0f / l;
-    uint16_t* op = a.o + ((int64_t)b * S + qrow) * a.ldo + (int64_t)h * HD;
-#pragma unroll
-    for (int i = 0; i < HD / 32; ++i)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const int hd = i * 32 + 8 * q4 + 4 * half;
-        store_bf16x4(op + hd, o[i][4 * q4] * inv_l, o[i][4 * q4 + 1] * inv_l, o[i][4 * q4 + 2] * inv_l,
-                     o[i][4 * q4 + 3] * inv_l);
-      }
-    if (half == 0) a.lse[((int64_t)b * H + h) * S + qrow] = (m + log2f(l)) * kLn2;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Backward, dK/dV pass.  256 threads; 128 keys per workgroup (32 per wave);
-// 64-query steps over every query head of the kv head's group.
-// ---------------------------------------------------------------------------
-template <int HD>
-__global__ void __launch_bounds__(256) attn_bwd_dkdv_kernel(AttnArgs a) {
-  constexpr int BKV = 128, BQ = 64, NT = 256;
-  constexpr int KROW = HD * 2 + 16;
-  constexpr int TROW = BQ * 2 + 8;
-  __shared__ __attribute__((aligned(16))) char smem[2 * BQ * KROW + 2 * HD * TROW + 2 * BQ * 4];
-  char* Qs = smem;
-  char* dOs = Qs + BQ * KROW;
-  char* Qts = dOs + BQ * KROW;
-  char* dOts = Qts + HD * TROW;
-  float* lse2s = reinterpret_cast<float*>(dOts + HD * TROW);
-  float* Ds = lse2s + BQ;
-
-  const int S = a.S, H = a.H, KV = a.KV, rep = H / KV;
-  int kvb, b, g;
-  key_block_coords(blockIdx.x, a.B, KV, kvb, b, g);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int half = lane >> 5, l32 = lane & 31;
-  const int k0 = kvb * BKV, kw0 = k0 + 32 * wave;
-  const int kvrow = kw0 + l32;
-  const float c = a.scale * kLog2e;
-
-  bf16x8_t kf[HD / 16], vf[HD / 16];
-  {
-    const int64_t r = (int64_t)b * S + min(kvrow, S - 1);
-    const uint16_t* kp = a.k + r * a.ldk + (int64_t)g * HD + 8 * half;
-    const uint16_t* vp = a.v + r * a.ldv + (int64_t)g * HD + 8 * half;
-#pragma unroll
-    for (int kk = 0; kk < HD / 16; ++kk) {
-      kf[kk] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(kp + kk * 16));
-      vf[kk] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(vp + kk * 16));
-    }
-  }
-  f32x16_t dk[HD / 32], dv[HD / 32];
-#pragma unroll
-  for (int i = 0; i < HD / 32; ++i)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      dk[i][r] = 0.f;
-      dv[i][r] = 0.f;
-    }
-
-  const int qstart = (k0 / BQ) * BQ;
-  for (int hq = 0; hq < rep; ++hq) {
-    const int h = g * rep + hq;
-    const uint16_t* qbase = a.q + (int64_t)b * S * a.ldq + (int64_t)h * HD;
-    const uint16_t* dobase = a.dout + (int64_t)b * S * a.lddo + (int64_t)h * HD;
-    const uint16_t* qtbase = a.qt + (int64_t)(b * H + h) * HD * S;
-    const uint16_t* dotbase = a.dot + (int64_t)(b * H + h) * HD * S;
-    const float* lsep = a.lse + (int64_t)(b * H + h) * S;
-    const float* dp_ = a.delta + (int64_t)(b * H + h) * S;
-    for (int q0 = qstart; q0 < S; q0 += BQ) {
-      load_rows<HD, BQ, NT>(Qs, KROW, qbase, a.ldq, q0, S, tid);
-      load_rows<HD, BQ, NT>(dOs, KROW, dobase, a.lddo, q0, S, tid);
-      load_trows<HD, BQ, NT>(Qts, TROW, qtbase, S, q0, tid);
-      load_trows<HD, BQ, NT>(dOts, TROW, dotbase, S, q0, tid);
-      if (tid < BQ) {
-        const int q = q0 + tid;
-        lse2s[tid] = q < S ? lsep[q] * kLog2e : 0.f;
-        Ds[tid] = q < S ? dp_[q] : 0.f;
-      }
-      __syncthreads();
-      if (q0 + BQ - 1 >= kw0 && kw0 < S) {
-        f32x16_t s[2], dp[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            s[t][r] = 0.f;
-            dp[t][r] = 0.f;
-          }
-#pragma unroll
-          for (int kk = 0; kk < HD / 16; ++kk) {
-            const bf16x8_t aq = lds_frag16(Qs + (t * 32 + l32) * KROW + kk * 32 + half * 16);
-            s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aq, kf[kk], s[t], 0, 0, 0);
-            const bf16x8_t ado = lds_frag16(dOs + (t * 32 + l32) * KROW + kk * 32 + half * 16);
-            dp[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ado, vf[kk], dp[t], 0, 0, 0);
-          }
-        }
-        // lane holds key column kvrow; query rows ql = t*32 + 8*(r/4) + 4*half + r%4
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int r4 = 0; r4 < 4; ++r4) {
-            const int qlb = t * 32 + 8 * r4 + 4 * half;
-            const float4 l4 = *reinterpret_cast<const float4*>(lse2s + qlb);
-            const float4 d4 = *reinterpret_cast<const float4*>(Ds + qlb);
-            const float lv[4] = {l4.x, l4.y, l4.z, l4.w};
-            const float dvv[4] = {d4.x, d4.y, d4.z, d4.w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int r = 4 * r4 + e;
-              const int q = q0 + qlb + e;
-              const bool ok = q < S && kvrow <= q && kvrow < S;
-              const float p = ok ? __builtin_amdgcn_exp2f(fmaf(s[t][r], c, -lv[e])) : 0.f;
-              dp[t][r] = p * (dp[t][r] - dvv[e]);
-              s[t][r] = p;
-            }
-          }
-#pragma unroll
-        for (int ks = 0; ks < BQ / 16; ++ks) {
-          const bf16x8_t pb = pack8(s[ks >> 1], 8 * (ks & 1));
-          const bf16x8_t dsb = pack8(dp[ks >> 1], 8 * (ks & 1));
-#pragma unroll
-          for (int i = 0; i < HD / 32; ++i) {
-            const char* dorow = dOts + (i * 32 + l32) * TROW;
-            const bf16x8_t ado = lds_frag_2x4(dorow + (16 * ks + 4 * half) * 2, dorow + (16 * ks + 8 + 4 * half) * 2);
-            dv[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ado, pb, dv[i], 0, 0, 0);
-            const char* qrow_ = Qts + (i * 32 + l32) * TROW;
-            const bf16x8_t aq = lds_frag_2x4(qrow_ + (16 * ks + 4 * half) * 2, qrow_ + (16 * ks + 8 + 4 * half) * 2);
-            dk[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aq, dsb, dk[i], 0, 0, 0);
-          }
-        }
-      }
-      __syncthreads();
-    }
-  }
-  if (kvrow < S) {
-    uint16_t* dkp = a.dk + ((int64_t)b * S + kvrow) * a.lddk + (int64_t)g * HD;
-    uint16_t* dvp = a.dv + ((int64_t)b * S + kvrow) * a.lddv + (int64_t)g * HD;
-    const bool rope = a.rcos != nullptr;
-    store_grad_row<HD>(dkp, dk, a.scale, half, rope ? a.rcos + (int64_t)kvrow * HD : nullptr,
-                       rope ? a.rsin + (int64_t)kvrow * HD : nullptr);
-    store_grad_row<HD>(dvp, dv, 1.0f, half, nullptr, nullptr);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Backward, dQ pass.  256 threads; 128 queries per workgroup; 64-key steps.
-// ---------------------------------------------------------------------------
-template <int HD>
-__global__ void __launch_bounds__(256) attn_bwd_dq_kernel(AttnArgs a) {
-  constexpr int BQ = 128, BKV = 64, NT = 256;
-  constexpr int KROW = HD * 2 + 16;
-  constexpr int TROW = BKV * 2 + 8;
-  __shared__ __attribute__((aligned(16))) char smem[2 * BKV * KROW + HD * TROW];
-  char* Ks = smem;
-  char* Vs = Ks + BKV * KROW;
-  char* Kts = Vs + BKV * KROW;
-
-  const int S = a.S, H = a.H, KV = a.KV;
-  const int nqb = (S + BQ - 1) / BQ;
-  int qb, b, h;
-  query_block_coords(blockIdx.x, nqb, a.B, H, KV, qb, b, h);
-  const int g = h / (H / KV);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int half = lane >> 5, l32 = lane & 31;
-  const int q0 = qb * BQ, qw0 = q0 + 32 * wave;
-  const int qrow = qw0 + l32;
-  const int qc = min(qrow, S - 1);
-  const float c = a.scale * kLog2e;
-
-  bf16x8_t qf[HD / 16], df[HD / 16];
-  {
-    const uint16_t* qp = a.q + ((int64_t)b * S + qc) * a.ldq + (int64_t)h * HD + 8 * half;
-    const uint16_t* dp_ = a.dout + ((int64_t)b * S + qc) * a.lddo + (int64_t)h * HD + 8 * half;
-#pragma unroll
-    for (int kk = 0; kk < HD / 16; ++kk) {
-      qf[kk] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(qp + kk * 16));
-      df[kk] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(dp_ + kk * 16));
-    }
-  }
-  const float lse2 = a.lse[((int64_t)b * H + h) * S + qc] * kLog2e;
-  const float Dq = a.delta[((int64_t)b * H + h) * S + qc];
-  f32x16_t dq[HD / 32];
-#pragma unroll
-  for (int i = 0; i < HD / 32; ++i)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) dq[i][r] = 0.f;
-
-  const int kv_end = min(S, q0 + BQ);
-  const int kv_end_w = min(S, qw0 + 32);
-  const uint16_t* kbase = a.k + (int64_t)b * S * a.ldk + (int64_t)g * HD;
-  const uint16_t* vbase = a.v + (int64_t)b * S * a.ldv + (int64_t)g * HD;
-  const uint16_t* ktbase = a.kt + (int64_t)(b * KV + g) * HD * S;
-
-  for (int k0 = 0; k0 < kv_end; k0 += BKV) {
-    load_rows<HD, BKV, NT>(Ks, KROW, kbase, a.ldk, k0, S, tid);
-    load_rows<HD, BKV, NT>(Vs, KROW, vbase, a.ldv, k0, S, tid);
-    load_trows<HD, BKV, NT>(Kts, TROW, ktbase, S, k0, tid);
-    __syncthreads();
-    if (k0 < kv_end_w) {
-      f32x16_t st[2], dpt[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          st[t][r] = 0.f;
-          dpt[t][r] = 0.f;
-        }
-#pragma unroll
-        for (int kk = 0; kk < HD / 16; ++kk) {
-          const bf16x8_t ak = lds_frag16(Ks + (t * 32 + l32) * KROW + kk * 32 + half * 16);
-          st[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ak, qf[kk], st[t], 0, 0, 0);
-          const bf16x8_t av = lds_frag16(Vs + (t * 32 + l32) * KROW + kk * 32 + half * 16);
-          dpt[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, df[kk], dpt[t], 0, 0, 0);
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int kv = k0 + t * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-          const bool ok = kv <= qrow && kv < S && qrow < S;
-          const float p = ok ? __builtin_amdgcn_exp2f(fmaf(st[t][r], c, -lse2)) : 0.f;
-          dpt[t][r] = p * (dpt[t][r] - Dq);
-        }
-#pragma unroll
-      for (int ks = 0; ks < BKV / 16; ++ks) {
-        const bf16x8_t dsb = pack8(dpt[ks >> 1], 8 * (ks & 1));
-#pragma unroll
-        for (int i = 0; i < HD / 32; ++i) {
-          const char* row = Kts + (i * 32 + l32) * TROW;
-          const bf16x8_t ak = lds_frag_2x4(row + (16 * ks + 4 * half) * 2, row + (16 * ks + 8 + 4 * half) * 2);
-          dq[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ak, dsb, dq[i], 0, 0, 0);
-        }
-      }
-    }
-    __syncthreads();
-  }
-  if (qrow < S) {
-    uint16_t* dqp = a.dq + ((int64_t)b * S + qrow) * a.lddq + (int64_t)h * HD;
-    const bool rope = a.rcos != nullptr;
-    store_grad_row<HD>(dqp, dq, a.scale, half, rope ? a.rcos + (int64_t)qrow * HD : nullptr,
-                       rope ? a.rsin + (int64_t)qrow * HD : nullptr);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Tile path (S a multiple of 64).  Every operand tile is a [64][HD] bf16 block
+// Tile path.  Every operand tile is a [64][HD] bf16 block
 // of a row-major source (Q, dO, K or V rows), copied into LDS by
 // buffer_load_dwordx4 ... lds with no staging registers, in unpadded rows whose
 // 16-byte chunks are XOR-swizzled by tswz().  Operands that the MFMAs need
@@ -669,27 +120,11 @@ __global__ void __launch_bounds__(256) attn_bwd_dq_kernel(AttnArgs a) {
 // same tiles with ds_read_b64_tr_b16: within each 16-lane group, lane 4j+q
 // points at row k0+j, columns n0+4q..n0+4q+3, and lane i receives column
 // n0+i, rows k0..k0+3.  So no transposed copy of any operand exists in HBM.
+// kRagged instances take sequences that are not a multiple of 64: rows past
+// the end are clamped in the loads and masked with the diagonal.
 // Two LDS stages: the tiles of step i+1 are issued right after the barrier
 // that opens step i (the barrier's fence waits for the loads of step i).
 // ---------------------------------------------------------------------------
-typedef short v4i16_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4i16_t* lds_v4i16_ptr;
-
-// Chunk swizzle of a tile row r: keeps the 16-byte reads of 16 consecutive
-// rows (row fragments) and the 8-byte transposed reads of 4 consecutive rows
-// x 64 bytes (one half-wave of ds_read_b64_tr_b16) on distinct banks of the
-// 64-bank LDS.
-template <int HD>
-__device__ __forceinline__ int tswz(int r) {
-  if constexpr (HD == 128) return ((r & 3) << 2) | ((r >> 2) & 3);
-  else return (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
-}
-
-template <int HD>
-__device__ __forceinline__ int toff(int r, int chunk) {
-  return r * (HD * 2) + ((chunk ^ tswz<HD>(r)) << 4);
-}
-
 // Raw buffer starting at a tile's first row (src is the same for every
 // lane): the DMA loads below take a 32-bit per-lane offset within the tile's
 // 64 rows, which measured faster than 64-bit per-lane addresses.
@@ -714,63 +149,45 @@ __device__ __forceinline__ void dma_tile(const uint16_t* src, int64_t ld, char* 
   }
 }
 
+// dma_tile with rows past `nvalid` (1..63) clamped to the last valid one;
+// their results are masked.
+template <int HD>
+__device__ __forceinline__ void dma_tile_tail(const uint16_t* src, int64_t ld, int nvalid, char* dst, int wave,
+                                              int lane) {
+  constexpr int kRowsPerLoad = 1024 / (HD * 2), kChunks = HD / 8;
+  constexpr int kPer = 64 / kRowsPerLoad / 4;
+  const lz_v4i rsrc = tile_rsrc(src);
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    const int r = (wave * kPer + q) * kRowsPerLoad + lane / kChunks;
+    const int c = (lane % kChunks) ^ tswz<HD>(r);
+    const uint32_t voff = (uint32_t)((min(r, nvalid - 1) * ld + c * 8) * 2);
+    if (q == 0) lz_dma16_first(rsrc, voff, 0, dst + (wave * kPer + q) * 1024);
+    else lds_dma16(rsrc, voff, dst + (wave * kPer + q) * 1024);
+  }
+}
+
+// The tile of rows r0 .. r0+63 of a sequence of S rows (kRagged: its last
+// rows may not exist).
+template <int HD, bool kRagged>
+__device__ __forceinline__ void dma_seq_tile(const uint16_t* base, int64_t ld, int r0, int S, char* dst, int wave,
+                                             int lane) {
+  const uint16_t* src = base + (int64_t)r0 * ld;
+  if constexpr (kRagged) {
+    if (S - r0 < 64) {
+      dma_tile_tail<HD>(src, ld, S - r0, dst, wave, lane);
+      return;
+    }
+  }
+  dma_tile<HD>(src, ld, dst, wave, lane);
+}
+
 // 64 floats at src into LDS at dst by lanes 0-15 of the calling wave, and 64
 // floats at src2 into dst + 256 by lanes 16-31 (src, src2 and dst uniform).
 __device__ __forceinline__ void dma_rows64(const float* src, const float* src2, char* dst, int lane) {
   if (lane < 16) lz_dma16(lz_buffer_rsrc(src), 16 * lane, 0, dst);
   else if (lane < 32) lz_dma16(lz_buffer_rsrc(src2), 16 * (lane - 16), 0, dst);
 }
-
-// Per-lane LDS offsets of the fragment reads of a tile.  tswz() depends only
-// on the row modulo 16, so every offset splits into a per-lane part and a
-// part that only depends on the 16-row block and the 32-column block.
-template <int HD>
-struct TileOffsets {
-  static constexpr int RB = HD * 2;
-  int row;              // row fragments: (lane % 32) * RB
-  int chunk[HD / 16];   // row fragments: ((2*kk + lane/32) ^ tswz) * 16
-  int tbase[2];         // transposed reads 1 and 2 (rows +0 and +8)
-  int tcol[HD / 32];    // transposed reads: 32-column block i
-
-  __device__ __forceinline__ void init(int lane) {
-    const int l32 = lane & 31, half = lane >> 5;
-    row = l32 * RB;
-    const int sw = tswz<HD>(l32);
-#pragma unroll
-    for (int kk = 0; kk < HD / 16; ++kk) chunk[kk] = ((2 * kk + half) ^ sw) << 4;
-    // lane 4j+q of each 16-lane group points at row r0 + j (+8), columns
-    // c0 + 16*(group % 2) + 4q .. +3
-    const int p = lane & 15;
-    const int col = ((lane >> 4) & 1) * 16 + 4 * (p & 3);
-    const int cl = col >> 3;
-    int swh = 0;
-#pragma unroll
-    for (int rd = 0; rd < 2; ++rd) {
-      const int r = 4 * half + (p >> 2) + 8 * rd;  // row within a 16-row block
-      const int swr = tswz<HD>(r);
-      tbase[rd] = r * RB + ((cl ^ (swr & 3)) << 4) + (col & 7) * 2;
-      swh = swr >> 2;  // the same for both reads
-    }
-#pragma unroll
-    for (int i = 0; i < HD / 32; ++i) tcol[i] = (i ^ swh) << 6;
-  }
-
-  // Row fragment: row 32*t + lane%32, columns 16*kk + 8*(lane/32) .. +7.
-  __device__ __forceinline__ bf16x8_t frag(const char* tile, int t, int kk) const {
-    return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(tile + t * 32 * RB + row + chunk[kk]));
-  }
-
-  // Transposed fragment for an MFMA operand whose k index runs over tile rows:
-  // lane l gets column 32*i + l%32 at rows 16*ks + 8*(e/4) + 4*(l/32) + e%4
-  // for k-slots e = 0..7 (the slot order of the accumulator layout).
-  __device__ __forceinline__ bf16x8_t frag_t(const char* tile, int ks, int i) const {
-    const char* blk = tile + ks * 16 * RB + tcol[i];
-    const v4i16_t x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(blk + tbase[0]));
-    const v4i16_t y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(blk + tbase[1]));
-    const uint2 xw = __builtin_bit_cast(uint2, x), yw = __builtin_bit_cast(uint2, y);
-    return __builtin_bit_cast(bf16x8_t, make_uint4(xw.x, xw.y, yw.x, yw.y));
-  }
-};
 
 // Forward on tiles: 128 queries per workgroup (32 per wave), 64-key steps,
 // K and V tiles double-buffered in LDS (the next step's tiles are issued
@@ -849,7 +266,7 @@ __device__ __forceinline__ void fwd_softmax_pv(f32x16_t (&s)[2], f32x16_t (&o)[H
   }
 }
 
-template <int HD, typename F>
+template <int HD, typename F, bool kRagged = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 4 : 2, HD == 64 ? 4 : 2))) attn_fwd_tile_kernel(AttnArgs a) {
   constexpr int BQ = 128, BKV = 64;
   constexpr int kTile = BKV * HD * 2;
@@ -884,27 +301,27 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 
   float m = -INFINITY, l = 0.f;
   const float c = a.scale * kLog2e;
 
-  const int kv_end = min(S, q0 + BQ);  // a multiple of 64
+  const int kv_end = min(S, q0 + BQ);  // a multiple of 64 unless kRagged
   const int kv_end_w = qw0 < S ? min(S, qw0 + 32) : 0;  // a wave past the sequence computes nothing
   const uint16_t* kbase = a.k + (int64_t)b * S * a.ldk + (int64_t)g * HD;
   const uint16_t* vbase = a.v + (int64_t)b * S * a.ldv + (int64_t)g * HD;
-  const int nsteps = kv_end / BKV;
+  const int nsteps = kRagged ? (kv_end + BKV - 1) / BKV : kv_end / BKV;
 
   // Step it: wait for its K/V (and every wave's reads of step it-1), then
   // issue step it+1's tiles into the other slot.
   auto open_step = [&](int it) {
     dma_barrier();
     if (it + 1 < nsteps) {
-      dma_tile<HD>(kbase + (int64_t)(it + 1) * BKV * a.ldk, a.ldk, Ks + ((it + 1) & 1) * kTile, wave, lane);
-      dma_tile<HD>(vbase + (int64_t)(it + 1) * BKV * a.ldv, a.ldv, Vs + ((it + 1) & 1) * kTile, wave, lane);
+      dma_seq_tile<HD, kRagged>(kbase, a.ldk, (it + 1) * BKV, S, Ks + ((it + 1) & 1) * kTile, wave, lane);
+      dma_seq_tile<HD, kRagged>(vbase, a.ldv, (it + 1) * BKV, S, Vs + ((it + 1) & 1) * kTile, wave, lane);
     }
   };
   // This wave's last step holds its diagonal (the only step with masked
   // keys: 32 queries starting at a multiple of 32 against 64-key steps);
   // the loop before it has no branch, so the accumulators stay in place.
   const int last_w = kv_end_w > 0 ? (kv_end_w - 1) / BKV : -1;
-  dma_tile<HD>(kbase, a.ldk, Ks, wave, lane);
-  dma_tile<HD>(vbase, a.ldv, Vs, wave, lane);
+  dma_seq_tile<HD, kRagged>(kbase, a.ldk, 0, S, Ks, wave, lane);
+  dma_seq_tile<HD, kRagged>(vbase, a.ldv, 0, S, Vs, wave, lane);
   int it = 0;
   for (; it < last_w; ++it) {
     open_step(it);
@@ -935,6 +352,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 
   }
 }
 
+// The same for rows of any alignment, of which nvalid exist (the rest repeat
+// the last one): 4 bytes per lane, one load per array.
+__device__ __forceinline__ void dma_rows64_any(const float* src, const float* src2, int nvalid, char* dst, int lane) {
+  const uint32_t voff = 4 * min(lane, nvalid - 1);
+  lz_dma4_first(lz_buffer_rsrc(src), voff, dst);
+  lz_dma4_first(lz_buffer_rsrc(src2), voff, dst + 256);
+}
+
 // A [64][HD] tile like dma_tile, loaded by the four waves of group `wg4`
 // (wave index 0..3 within the group), rows past `nvalid` clamped to the last
 // valid row (their results are masked).
@@ -954,7 +379,7 @@ __device__ __forceinline__ void dma_tile_rows(const uint16_t* src, int64_t ld, i
 
 // Issues the tiles of dK/dV step `step` for the 8-wave kernel: Q by waves
 // 0-3, dO by waves 4-7, lse and delta by wave 0.
-template <int HD>
+template <int HD, bool kRagged>
 __device__ __forceinline__ void dkdv8_issue(const AttnArgs& a, int step, int nqs, int qstart, int b, int g, int rep,
                                             char* st, int wave, int lane) {
   constexpr int kTile = 64 * HD * 2;
@@ -962,12 +387,14 @@ __device__ __forceinline__ void dkdv8_issue(const AttnArgs& a, int step, int nqs
   const int hq = step / nqs, q0 = qstart + (step - hq * nqs) * 64;
   const int h = g * rep + hq;
   if (wave < 4)
-    dma_tile<HD>(a.q + ((int64_t)b * S + q0) * a.ldq + (int64_t)h * HD, a.ldq, st, wave, lane);
+    dma_seq_tile<HD, kRagged>(a.q + (int64_t)b * S * a.ldq + (int64_t)h * HD, a.ldq, q0, S, st, wave, lane);
   else
-    dma_tile<HD>(a.dout + ((int64_t)b * S + q0) * a.lddo + (int64_t)h * HD, a.lddo, st + kTile, wave - 4, lane);
+    dma_seq_tile<HD, kRagged>(a.dout + (int64_t)b * S * a.lddo + (int64_t)h * HD, a.lddo, q0, S, st + kTile, wave - 4,
+                              lane);
   if (wave == 0) {
     const int64_t off = ((int64_t)b * a.H + h) * S + q0;
-    dma_rows64(a.lse + off, a.delta + off, st + 2 * kTile, lane);
+    if constexpr (kRagged) dma_rows64_any(a.lse + off, a.delta + off, min(64, S - q0), st + 2 * kTile, lane);
+    else dma_rows64(a.lse + off, a.delta + off, st + 2 * kTile, lane);
   }
 }
 
@@ -979,12 +406,13 @@ __device__ __forceinline__ void dkdv8_issue(const AttnArgs& a, int step, int nqs
 // dK += dS^T Q from transposed LDS reads.
 // One 64-query step of the 8-wave dK/dV kernel for this wave's 32 keys:
 // S^T and dP^T, P and dS, then dV += P^T dO and dK += dS^T Q.  MASK: the
-// step crosses this wave's diagonal, so pairs with key > query are dropped
-// (the other steps carry no masking instructions).
-template <int HD, bool MASK, typename F>
+// step crosses this wave's diagonal (or the sequence's end), so pairs with
+// key > query (or query >= S) are dropped; the other steps carry no masking
+// instructions.
+template <int HD, bool MASK, typename F, bool kRagged>
 __device__ __forceinline__ void dkdv_step(f32x16_t (&dk)[HD / 32], f32x16_t (&dv)[HD / 32], const TileOffsets<HD>& to,
                                           const char* Qt, const char* Vt, const bf16x8_t (&kf)[HD / 16], float c,
-                                          int q0, int kvrow, int wave, int half) {
+                                          int q0, int kvrow, int S, int wave, int half) {
   constexpr int kTile = 64 * HD * 2;
   const char* dOt = Qt + kTile;
   const float* lse_s = reinterpret_cast<const float*>(Qt + 2 * kTile);
@@ -1017,7 +445,10 @@ __device__ __forceinline__ void dkdv_step(f32x16_t (&dk)[HD / 32], f32x16_t (&dv
       for (int e = 0; e < 4; ++e) {
         const int r = 4 * r4 + e;
         float p = __builtin_amdgcn_exp2f(fmaf(sc[r], c, -lv[e] * kLog2e));
-        if constexpr (MASK) p = kvrow <= q0 + qlb + e ? p : 0.f;
+        if constexpr (MASK) {
+          p = kvrow <= q0 + qlb + e ? p : 0.f;
+          if constexpr (kRagged) p = q0 + qlb + e < S ? p : 0.f;
+        }
         dp[r] = p * (dp[r] - dvv[e]);
         sc[r] = p;
       }
@@ -1037,7 +468,7 @@ __device__ __forceinline__ void dkdv_step(f32x16_t (&dk)[HD / 32], f32x16_t (&dv
   }
 }
 
-template <int HD, typename F>
+template <int HD, typename F, bool kRagged = false>
 __global__ void __launch_bounds__(512) attn_bwd_dkdv_wide_kernel(AttnArgs a) {
   constexpr int BKV = 256, BQ = 64;
   constexpr int kTile = BQ * HD * 2;
@@ -1086,12 +517,12 @@ __global__ void __launch_bounds__(512) attn_bwd_dkdv_wide_kernel(AttnArgs a) {
     }
 
   const int qstart = (k0 / BQ) * BQ;
-  const int nqs = (S - qstart) / BQ;
+  const int nqs = kRagged ? (S - qstart + BQ - 1) / BQ : (S - qstart) / BQ;
   const int nsteps = rep * nqs;
   auto open_step = [&](int step) {
     dma_barrier();  // this step's tiles (and the V tile) landed, last step's reads retired
     if (step + 1 < nsteps)
-      dkdv8_issue<HD>(a, step + 1, nqs, qstart, b, g, rep, stages + ((step + 1) & 1) * kStage, wave, lane);
+      dkdv8_issue<HD, kRagged>(a, step + 1, nqs, qstart, b, g, rep, stages + ((step + 1) & 1) * kStage, wave, lane);
   };
   // Per query head, the 64-query blocks j = 0 .. nqs-1 (queries qstart + 64j
   // on) fall into three runs for this wave's keys kw0 .. kw0+31 (kw0 a
@@ -1101,18 +532,28 @@ __global__ void __launch_bounds__(512) attn_bwd_dkdv_wide_kernel(AttnArgs a) {
   const int rel = kw0 - qstart;  // 0 .. 224
   const int j_first = kw0 < S ? min(nqs, rel / BQ) : nqs;
   const int j_unmasked = kw0 < S ? min(nqs, (rel + 32 + BQ - 1) / BQ) : nqs;
-  dkdv8_issue<HD>(a, 0, nqs, qstart, b, g, rep, stages, wave, lane);
+  const int j_tail = kRagged && S % BQ && kw0 < S ? max(j_unmasked, nqs - 1) : nqs;  // a last block of fewer queries
+  dkdv8_issue<HD, kRagged>(a, 0, nqs, qstart, b, g, rep, stages, wave, lane);
   int step = 0;
   for (int hq = 0; hq < rep; ++hq) {
     int j = 0;
     for (; j < j_first; ++j, ++step) open_step(step);
     for (; j < j_unmasked; ++j, ++step) {
       open_step(step);
-      dkdv_step<HD, true, F>(dk, dv, to, stages + (step & 1) * kStage, Vt, kf, c, qstart + j * BQ, kvrow, wave, half);
+      dkdv_step<HD, true, F, kRagged>(dk, dv, to, stages + (step & 1) * kStage, Vt, kf, c, qstart + j * BQ, kvrow, S,
+                                      wave, half);
     }
-    for (; j < nqs; ++j, ++step) {
+    for (; j < j_tail; ++j, ++step) {
       open_step(step);
-      dkdv_step<HD, false, F>(dk, dv, to, stages + (step & 1) * kStage, Vt, kf, c, qstart + j * BQ, kvrow, wave, half);
+      dkdv_step<HD, false, F, kRagged>(dk, dv, to, stages + (step & 1) * kStage, Vt, kf, c, qstart + j * BQ, kvrow, S,
+                                       wave, half);
+    }
+    if constexpr (kRagged) {
+      for (; j < nqs; ++j, ++step) {
+        open_step(step);
+        dkdv_step<HD, true, F, true>(dk, dv, to, stages + (step & 1) * kStage, Vt, kf, c, qstart + j * BQ, kvrow, S,
+                                     wave, half);
+      }
     }
   }
   if (kvrow < S) {
@@ -1179,7 +620,7 @@ __device__ __forceinline__ void dq_step(f32x16_t (&dq)[HD / 32], const TileOffse
 // (from the dO fragments held in registers and the same columns of O, a.o)
 // and written to a.delta_w for the dK/dV kernel that runs next, instead of
 // read from a.delta.
-template <int HD, typename F, bool kDelta = false>
+template <int HD, typename F, bool kDelta = false, bool kRagged = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) attn_bwd_dq_tile_kernel(AttnArgs a) {
   constexpr int BQ = 128, BKV = 64;
   constexpr int kTile = BKV * HD * 2;
@@ -1243,21 +684,21 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int kv_end_w = qw0 < S ? min(S, qw0 + 32) : 0;  // a wave past the sequence computes nothing
   const uint16_t* kbase = a.k + (int64_t)b * S * a.ldk + (int64_t)g * HD;
   const uint16_t* vbase = a.v + (int64_t)b * S * a.ldv + (int64_t)g * HD;
-  const int nsteps = kv_end / BKV;
+  const int nsteps = kRagged ? (kv_end + BKV - 1) / BKV : kv_end / BKV;
 
   auto open_step = [&](int it) {
     dma_barrier();  // this step's tiles landed (every wave's loads), last step's reads retired
     if (it + 1 < nsteps) {
       char* nxt = smem + ((it + 1) & 1) * kStage;
-      dma_tile<HD>(kbase + (int64_t)(it + 1) * BKV * a.ldk, a.ldk, nxt, wave, lane);
-      dma_tile<HD>(vbase + (int64_t)(it + 1) * BKV * a.ldv, a.ldv, nxt + kTile, wave, lane);
+      dma_seq_tile<HD, kRagged>(kbase, a.ldk, (it + 1) * BKV, S, nxt, wave, lane);
+      dma_seq_tile<HD, kRagged>(vbase, a.ldv, (it + 1) * BKV, S, nxt + kTile, wave, lane);
     }
   };
   // This wave's last step holds its diagonal (the only masked step); the
   // steps after it only join the barriers.
   const int last_w = kv_end_w > 0 ? (kv_end_w - 1) / BKV : -1;
-  dma_tile<HD>(kbase, a.ldk, smem, wave, lane);
-  dma_tile<HD>(vbase, a.ldv, smem + kTile, wave, lane);
+  dma_seq_tile<HD, kRagged>(kbase, a.ldk, 0, S, smem, wave, lane);
+  dma_seq_tile<HD, kRagged>(vbase, a.ldv, 0, S, smem + kTile, wave, lane);
   int it = 0;
   for (; it < last_w; ++it) {
     open_step(it);
@@ -1332,9 +773,9 @@ __global__ void __launch_bounds__(256) attn_delta_vec_kernel(const uint16_t* __r
 }
 
 // ---------------------------------------------------------------------------
-// Generic path (any even head dim up to 256, bf16 or fp32): one wave per
-// query row (forward, dQ) or key row (dK/dV), lanes split the head dim, fp32
-// online softmax.  Used where the MFMA tiling does not apply.
+// Generic path (any even head dim up to 256, any dtype and alignment): one
+// wave per query row (forward, dQ) or key row (dK/dV), lanes split the head
+// dim, fp32 online softmax.  Used where neither MFMA family applies.
 // ---------------------------------------------------------------------------
 template <typename T>
 struct GenArgs {
@@ -1563,7 +1004,8 @@ __global__ void __launch_bounds__(256) attn_bwd_dkdv_generic_kernel(GenArgs<T> a
 }
 
 // ---------------------------------------------------------------------------
-// Small head dims (16, 32): four lanes (a quad) per query row (forward, dQ)
+// Small head dims (16, and 32 where the rows are not aligned for the
+// wave-private kernels of attn_wave.hip): four lanes (a quad) per query row (forward, dQ)
 // or key row (dK/dV), each holding a quarter of that row, its accumulators
 // and the row's running softmax in registers; a workgroup of four waves owns
 // 64 rows.  The other side's rows pass through LDS 64 at a time as fp32
@@ -1839,19 +1281,162 @@ int check_shape(int64_t B, int64_t S, int64_t H, int64_t KV, int64_t hd) {
   return LZ_OK;
 }
 
+LzWaveArgs wave_fwd_args(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, void* o,
+                         int64_t ldo, float* lse, int64_t B, int64_t S, int64_t H, int64_t KV, float scale) {
+  LzWaveArgs a{};
+  a.q = q; a.k = k; a.v = v;
+  a.ldq = ldq; a.ldk = ldk; a.ldv = ldv;
+  a.o = o; a.ldo = ldo; a.lse = lse;
+  a.B = (int)B; a.S = (int)S; a.H = (int)H; a.KV = (int)KV; a.scale = scale;
+  return a;
+}
+
+void wave_bwd_args(LzWaveArgs& a, const void* dout, int64_t lddo, const float* delta, void* dq, int64_t lddq, void* dk,
+                   int64_t lddk, void* dv, int64_t lddv) {
+  a.dout = dout; a.lddo = lddo; a.delta = delta;
+  a.dq = dq; a.dk = dk; a.dv = dv;
+  a.lddq = lddq; a.lddk = lddk; a.lddv = lddv;
+}
+
+// Where the tile kernels' workgroups are too few to fill the chip the
+// wave-private kernels (a quarter or an eighth of the rows per workgroup, the
+// other side split over its waves) are faster; `wgs` is the tile kernel's
+// grid.  Lines drawn from both sides at B 1..8, S 128..2048, heads 12/4 and
+// 32/8 of 64 and 16/8 of 128 (us, tile / wave):
+//   forward, hd 64: 96 workgroups S 1024 16.1 / 11.5, S 512 10.0 / 8.8,
+//     S 256 7.0 / 7.6; 192 at S 2048 28.4 / 26.8, S 1024 16.7 / 18.4; hd 128: 64
+//     at S 512 13.8 / 12.0, 112 at S 777 19.7 / 19.1, 128 at S 1024 24.1 / 25.0
+//   dQ gains 1-5 us up to 64 workgroups, and at 96-128 where S >= 768
+//   dK/dV (256 keys and every query head of the group per tile workgroup):
+//     hd 64: 32 workgroups 109 / 43 for the whole backward, 192 at S 1536
+//     194 / 181, 256 at S 1024 204 / 226; hd 128: 64 at S 1024 134 / 82, 128 at
+//     S 2048 260 / 235 and S 777 144 / 101, at S 512 86 / 91
+bool wave_fwd_better(int64_t hd, int64_t S, int64_t wgs) {
+  if (wgs <= 64) return true;
+  if (hd == 64) return (wgs <= 96 && S > 256) || (wgs <= 192 && S > 1024);
+  return wgs <= 112 && S >= 768;
+}
+bool wave_dq_better(int64_t S, int64_t wgs) { return wgs <= 64 || (wgs <= 128 && S >= 768); }
+bool wave_dkdv_better(int64_t hd, int64_t S, int64_t wgs) {
+  if (hd == 64) return wgs <= 192;
+  return wgs < 128 || (wgs == 128 && (S > 512 || S % 64));
+}
+
+// The forward of 16-bit causal attention with head dim 64 or 128 (aligned as
+// mfma_ok asks; fp16: S a multiple of 64).
+int tiles_fwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, void* o, int64_t ldo,
+              float* lse, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t hd, float scale, int dtype,
+              hipStream_t s) {
+  const int64_t grid = lz_cdiv(S, 128) * B * H;
+  if (dtype == LZ_BF16 && wave_fwd_better(hd, S, grid)) {
+    const LzWaveArgs w = wave_fwd_args(q, ldq, k, ldk, v, ldv, o, ldo, lse, B, S, H, KV, scale);
+    if (lz_attn_wave_ok(w, dtype, hd, false)) return lz_attn_wave_pass(w, dtype, hd, kWaveRounded, kWaveFwd, s);
+  }
+  AttnArgs a{};
+  a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v;
+  a.ldq = ldq; a.ldk = ldk; a.ldv = ldv;
+  a.o = (uint16_t*)o; a.ldo = ldo; a.lse = lse;
+  a.B = (int)B; a.S = (int)S; a.H = (int)H; a.KV = (int)KV; a.scale = scale;
+  const unsigned g = (unsigned)grid;
+  if (dtype == LZ_F16) {
+    if (hd == 128) attn_fwd_tile_kernel<128, FmtF16><<<g, 256, 0, s>>>(a);
+    else attn_fwd_tile_kernel<64, FmtF16><<<g, 256, 0, s>>>(a);
+  } else if (S % 64) {
+    if (hd == 128) attn_fwd_tile_kernel<128, FmtBF16, true><<<g, 256, 0, s>>>(a);
+    else attn_fwd_tile_kernel<64, FmtBF16, true><<<g, 256, 0, s>>>(a);
+  } else {
+    if (hd == 128) attn_fwd_tile_kernel<128, FmtBF16><<<g, 256, 0, s>>>(a);
+    else attn_fwd_tile_kernel<64, FmtBF16><<<g, 256, 0, s>>>(a);
+  }
+  return lz_check_launch("lz_attn_fwd");
+}
+
+template <int HD, typename F, bool kRagged>
+void launch_dq_tiles(const AttnArgs& a, hipStream_t s) {
+  const unsigned grid = (unsigned)(lz_cdiv(a.S, 128) * a.B * a.H);
+  if (a.delta_w) attn_bwd_dq_tile_kernel<HD, F, true, kRagged><<<grid, 256, 0, s>>>(a);
+  else attn_bwd_dq_tile_kernel<HD, F, false, kRagged><<<grid, 256, 0, s>>>(a);
+}
+
+template <int HD, typename F, bool kRagged>
+void launch_dkdv_tiles(const AttnArgs& a, hipStream_t s) {
+  const unsigned grid = (unsigned)(lz_cdiv(a.S, 256) * a.B * a.KV);
+  attn_bwd_dkdv_wide_kernel<HD, F, kRagged><<<grid, 512, 0, s>>>(a);
+}
+
+// Its backward, with delta given or (delta_w) formed from o.
+int tiles_bwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, const void* dout,
+              int64_t lddo, const float* lse, const float* delta, void* dq, int64_t lddq, void* dk, int64_t lddk,
+              void* dv, int64_t lddv, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t hd, float scale,
+              const void* rope_cos, const void* rope_sin, int dtype, hipStream_t s, bool& rope_done, const void* o,
+              int64_t ldo, float* delta_w) {
+  AttnArgs a{};
+  a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v;
+  a.ldq = ldq; a.ldk = ldk; a.ldv = ldv;
+  a.lse = const_cast<float*>(lse);
+  a.dout = (const uint16_t*)dout; a.lddo = lddo;
+  a.o = (uint16_t*)const_cast<void*>(o); a.ldo = ldo;
+  a.delta_w = delta_w; a.delta = delta_w ? delta_w : delta;
+  a.dq = (uint16_t*)dq; a.dk = (uint16_t*)dk; a.dv = (uint16_t*)dv;
+  a.lddq = lddq; a.lddk = lddk; a.lddv = lddv;
+  a.rcos = (const uint16_t*)rope_cos; a.rsin = (const uint16_t*)rope_sin;
+  a.B = (int)B; a.S = (int)S; a.H = (int)H; a.KV = (int)KV; a.scale = scale;
+  LzWaveArgs w = wave_fwd_args(q, ldq, k, ldk, v, ldv, const_cast<void*>(o), ldo, const_cast<float*>(lse), B, S, H, KV,
+                               scale);
+  wave_bwd_args(w, dout, lddo, delta, dq, lddq, dk, lddk, dv, lddv);
+  w.delta_w = delta_w;
+  const bool can_wave = dtype == LZ_BF16 && lz_attn_wave_ok(w, dtype, hd, true);
+  const bool wave_dq = can_wave && wave_dq_better(S, lz_cdiv(S, 128) * B * H);
+  const bool wave_dkdv = can_wave && wave_dkdv_better(hd, S, lz_cdiv(S, 256) * B * KV);
+  rope_done = !wave_dq && !wave_dkdv;  // only the tile kernels rotate; the caller rotates after the others
+  if (!rope_done) a.rcos = a.rsin = nullptr;
+  // dQ first: it forms the delta that dK/dV reads when delta_w is set
+  if (wave_dq) {
+    const int rc = lz_attn_wave_pass(w, dtype, hd, kWaveRounded, kWaveDq, s);
+    if (rc) return rc;
+  } else if (dtype == LZ_F16) {
+    if (hd == 128) launch_dq_tiles<128, FmtF16, false>(a, s);
+    else launch_dq_tiles<64, FmtF16, false>(a, s);
+  } else if (S % 64) {
+    if (hd == 128) launch_dq_tiles<128, FmtBF16, true>(a, s);
+    else launch_dq_tiles<64, FmtBF16, true>(a, s);
+  } else {
+    if (hd == 128) launch_dq_tiles<128, FmtBF16, false>(a, s);
+    else launch_dq_tiles<64, FmtBF16, false>(a, s);
+  }
+  int rc = lz_check_launch("lz_attn_bwd");
+  if (rc) return rc;
+  if (wave_dkdv) {
+    if (delta_w) w.delta = delta_w;
+    return lz_attn_wave_pass(w, dtype, hd, kWaveRounded, kWaveDkdv, s);
+  }
+  if (dtype == LZ_F16) {
+    if (hd == 128) launch_dkdv_tiles<128, FmtF16, false>(a, s);
+    else launch_dkdv_tiles<64, FmtF16, false>(a, s);
+  } else if (S % 64) {
+    if (hd == 128) launch_dkdv_tiles<128, FmtBF16, true>(a, s);
+    else launch_dkdv_tiles<64, FmtBF16, true>(a, s);
+  } else {
+    if (hd == 128) launch_dkdv_tiles<128, FmtBF16, false>(a, s);
+    else launch_dkdv_tiles<64, FmtBF16, false>(a, s);
+  }
+  return lz_check_launch("lz_attn_bwd");
+}
+
 }  // namespace
 
-// Which path lz_attn_fwd/bwd take for these arguments: 2 = MFMA on LDS tiles
-// (S a multiple of 64; no transposed buffers), 1 = MFMA with the transposed
-// operand buffers (V^T for the forward; Q^T, K^T, dO^T for the backward),
-// 0 = generic.  fp16 takes the tile path or the generic one.
+// What lz_attn_fwd/bwd take for these arguments: 2 = MFMA on LDS tiles (S a
+// multiple of 64; no transposed buffers), 1 = the same dtypes and head dims at
+// other lengths, for which lz_attn_fwd/bwd ask for transposed operand buffers
+// (V^T; Q^T, K^T, dO^T: required, no longer read) and lz_attn_fwd_direct /
+// lz_attn_bwd_direct do not, 0 = the rest.
 LZ_EXPORT int lz_attn_path(int dtype, int64_t S, int64_t hd, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo) {
   const bool mfma = (dtype == LZ_BF16 || (dtype == LZ_F16 && S % 64 == 0)) && (hd == 64 || hd == 128) &&
                     strides_ok(ldq, ldk, ldv, ldo);
   return mfma ? (S % 64 == 0 ? 2 : 1) : 0;
 }
 
-// Forward.  vt: V^T [B,KV,hd,S] (needed on the MFMA path only).
+// Forward.  vt: V^T [B,KV,hd,S] (required where lz_attn_path is 1).
 LZ_EXPORT int lz_attn_fwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
                           const void* vt, void* o, int64_t ldo, float* lse, int64_t B, int64_t S, int64_t H, int64_t KV,
                           int64_t hd, float scale, int dtype, void* stream) {
@@ -1859,34 +1444,14 @@ LZ_EXPORT int lz_attn_fwd(const void* q, int64_t ldq, const void* k, int64_t ldk
   if (rc) return rc;
   LZ_REQUIRE(q && k && v && o && lse, "lz_attn_fwd: null pointer");
   hipStream_t s = lz_stream(stream);
-  if (mfma_ok(dtype, hd, ldq, ldk, ldv, ldo, q, k, v, o) && S % 64 == 0) {
-    AttnArgs a{};
-    a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v;
-    a.ldq = ldq; a.ldk = ldk; a.ldv = ldv;
-    a.o = (uint16_t*)o; a.ldo = ldo; a.lse = lse;
-    a.B = (int)B; a.S = (int)S; a.H = (int)H; a.KV = (int)KV; a.scale = scale;
-    const unsigned grid = (unsigned)(lz_cdiv(S, 128) * B * H);
-    if (dtype == LZ_F16) {
-      if (hd == 128) attn_fwd_tile_kernel<128, FmtF16><<<grid, 256, 0, s>>>(a);
-      else attn_fwd_tile_kernel<64, FmtF16><<<grid, 256, 0, s>>>(a);
-    } else {
-      if (hd == 128) attn_fwd_tile_kernel<128, FmtBF16><<<grid, 256, 0, s>>>(a);
-      else attn_fwd_tile_kernel<64, FmtBF16><<<grid, 256, 0, s>>>(a);
-    }
-    return lz_check_launch("lz_attn_fwd");
+  const bool mfma = mfma_ok(dtype, hd, ldq, ldk, ldv, ldo, q, k, v, o);
+  if (mfma && S % 64 == 0) return tiles_fwd(q, ldq, k, ldk, v, ldv, o, ldo, lse, B, S, H, KV, hd, scale, dtype, s);
+  if (mfma && dtype == LZ_BF16) {
+    LZ_REQUIRE(vt && lz_aligned16(vt), "lz_attn_fwd: this shape takes an aligned V^T buffer");
+    return tiles_fwd(q, ldq, k, ldk, v, ldv, o, ldo, lse, B, S, H, KV, hd, scale, dtype, s);
   }
-  if (dtype == LZ_BF16 && mfma_ok(dtype, hd, ldq, ldk, ldv, ldo, q, k, v, o)) {
-    LZ_REQUIRE(vt && lz_aligned16(vt), "lz_attn_fwd: MFMA path needs an aligned V^T buffer");
-    AttnArgs a{};
-    a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v;
-    a.ldq = ldq; a.ldk = ldk; a.ldv = ldv;
-    a.o = (uint16_t*)o; a.ldo = ldo; a.lse = lse; a.vt = (const uint16_t*)vt;
-    a.B = (int)B; a.S = (int)S; a.H = (int)H; a.KV = (int)KV; a.scale = scale;
-    const unsigned grid = (unsigned)(lz_cdiv(S, 128) * B * H);
-    if (hd == 128) attn_fwd_kernel<128><<<grid, 256, 0, s>>>(a);
-    else attn_fwd_kernel<64><<<grid, 256, 0, s>>>(a);
-    return lz_check_launch("lz_attn_fwd");
-  }
+  const LzWaveArgs w = wave_fwd_args(q, ldq, k, ldk, v, ldv, o, ldo, lse, B, S, H, KV, scale);
+  if (lz_attn_wave_ok(w, dtype, hd, false)) return lz_attn_wave_pass(w, dtype, hd, kWaveSplit, kWaveFwd, s);
   const unsigned grid = (unsigned)lz_cdiv(B * H * S, 4);
   if (dtype == LZ_BF16) {
     GenArgs<uint16_t> a{};
@@ -1955,8 +1520,8 @@ int attn_bwd_impl(const void* q, int64_t ldq, const void* k, int64_t ldk, const 
 
 }  // namespace
 
-// Backward.  On the MFMA path qt [B,H,hd,S], kt [B,KV,hd,S] and dot [B,H,hd,S]
-// are required; delta comes from lz_attn_delta.  dq/dk/dv are written (not
+// Backward.  Where lz_attn_path is 1 qt [B,H,hd,S], kt [B,KV,hd,S] and dot
+// [B,H,hd,S] are required; delta comes from lz_attn_delta.  dq/dk/dv are written (not
 // accumulated).  rope_cos/rope_sin (both or neither; tables [>= S, hd] in the
 // activation dtype, row = position, as lz_rope takes): dq and dk come back
 // as the gradients of q and k before RoPE, i.e. with lz_rope's backward
@@ -2002,9 +1567,13 @@ LZ_EXPORT int lz_attn_bwd_with_o(const void* q, int64_t ldq, const void* k, int6
                                                         reinterpret_cast<uintptr_t>(rope_sin)) & 7) == 0),
              "lz_attn_bwd_with_o: RoPE needs an even head dim and 8-byte aligned tables");
   bool rope_done = false;
-  return attn_bwd_impl(q, ldq, k, ldk, v, ldv, dout, lddo, lse, delta, nullptr, nullptr, nullptr, dq, lddq, dk, lddk,
-                       dv, lddv, B, S, H, KV, hd, scale, rope_cos, rope_sin, dtype, lz_stream(stream), rope_done, o,
-                       ldo, delta);
+  rc = attn_bwd_impl(q, ldq, k, ldk, v, ldv, dout, lddo, lse, delta, nullptr, nullptr, nullptr, dq, lddq, dk, lddk, dv,
+                     lddv, B, S, H, KV, hd, scale, rope_cos, rope_sin, dtype, lz_stream(stream), rope_done, o, ldo,
+                     delta);
+  if (rc || rope_cos == nullptr || rope_done) return rc;
+  rc = lz_rope(dq, dtype, lddq, B * S, S, H, hd, rope_cos, rope_sin, 0, 1, stream);
+  if (rc) return rc;
+  return lz_rope(dk, dtype, lddk, B * S, S, KV, hd, rope_cos, rope_sin, 0, 1, stream);
 }
 
 namespace {
@@ -2018,84 +1587,14 @@ int attn_bwd_impl(const void* q, int64_t ldq, const void* k, int64_t ldk, const 
                     lddv % 4 == 0;
   LZ_REQUIRE(delta_w == nullptr || (mfma && S % 64 == 0),
              "lz_attn_bwd_with_o: this shape takes the other kernels (use lz_attn_delta + lz_attn_bwd)");
-  if (mfma && S % 64 == 0) {
-    AttnArgs a{};
-    a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v;
-    a.ldq = ldq; a.ldk = ldk; a.ldv = ldv;
-    a.lse = const_cast<float*>(lse);
-    a.dout = (const uint16_t*)dout; a.lddo = lddo; a.delta = delta;
-    a.dq = (uint16_t*)dq; a.dk = (uint16_t*)dk; a.dv = (uint16_t*)dv;
-    a.lddq = lddq; a.lddk = lddk; a.lddv = lddv;
-    a.rcos = (const uint16_t*)rope_cos; a.rsin = (const uint16_t*)rope_sin;
-    rope_done = true;
-    a.B = (int)B; a.S = (int)S; a.H = (int)H; a.KV = (int)KV; a.scale = scale;
-    const unsigned grid_kv = (unsigned)(lz_cdiv(S, 256) * B * KV);
-    const unsigned grid_q = (unsigned)(lz_cdiv(S, 128) * B * H);
-    if (delta_w) {
-      // the dQ pass computes delta (rowsum(dO * O)) and runs first; dK/dV reads it
-      a.o = (uint16_t*)const_cast<void*>(o);
-      a.ldo = ldo;
-      a.delta_w = delta_w;
-      a.delta = delta_w;
-      if (dtype == LZ_F16) {
-        if (hd == 128) attn_bwd_dq_tile_kernel<128, FmtF16, true><<<grid_q, 256, 0, s>>>(a);
-        else attn_bwd_dq_tile_kernel<64, FmtF16, true><<<grid_q, 256, 0, s>>>(a);
-      } else {
-        if (hd == 128) attn_bwd_dq_tile_kernel<128, FmtBF16, true><<<grid_q, 256, 0, s>>>(a);
-        else attn_bwd_dq_tile_kernel<64, FmtBF16, true><<<grid_q, 256, 0, s>>>(a);
-      }
-      const int rc = lz_check_launch("lz_attn_bwd_with_o");
-      if (rc) return rc;
-      if (dtype == LZ_F16) {
-        if (hd == 128) attn_bwd_dkdv_wide_kernel<128, FmtF16><<<grid_kv, 512, 0, s>>>(a);
-        else attn_bwd_dkdv_wide_kernel<64, FmtF16><<<grid_kv, 512, 0, s>>>(a);
-      } else {
-        if (hd == 128) attn_bwd_dkdv_wide_kernel<128, FmtBF16><<<grid_kv, 512, 0, s>>>(a);
-        else attn_bwd_dkdv_wide_kernel<64, FmtBF16><<<grid_kv, 512, 0, s>>>(a);
-      }
-      return lz_check_launch("lz_attn_bwd_with_o");
-    }
-    if (dtype == LZ_F16) {
-      if (hd == 128) {
-        attn_bwd_dkdv_wide_kernel<128, FmtF16><<<grid_kv, 512, 0, s>>>(a);
-        attn_bwd_dq_tile_kernel<128, FmtF16><<<grid_q, 256, 0, s>>>(a);
-      } else {
-        attn_bwd_dkdv_wide_kernel<64, FmtF16><<<grid_kv, 512, 0, s>>>(a);
-        attn_bwd_dq_tile_kernel<64, FmtF16><<<grid_q, 256, 0, s>>>(a);
-      }
-    } else if (hd == 128) {
-      attn_bwd_dkdv_wide_kernel<128, FmtBF16><<<grid_kv, 512, 0, s>>>(a);
-      attn_bwd_dq_tile_kernel<128, FmtBF16><<<grid_q, 256, 0, s>>>(a);
-    } else {
-      attn_bwd_dkdv_wide_kernel<64, FmtBF16><<<grid_kv, 512, 0, s>>>(a);
-      attn_bwd_dq_tile_kernel<64, FmtBF16><<<grid_q, 256, 0, s>>>(a);
-    }
-    return lz_check_launch("lz_attn_bwd");
-  }
-  if (mfma && dtype == LZ_BF16) {
-    LZ_REQUIRE(qt && kt && dot, "lz_attn_bwd: MFMA path needs the transposed Q, K and dO buffers");
-    AttnArgs a{};
-    a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v;
-    a.ldq = ldq; a.ldk = ldk; a.ldv = ldv;
-    a.lse = const_cast<float*>(lse);
-    a.qt = (const uint16_t*)qt; a.kt = (const uint16_t*)kt; a.dout = (const uint16_t*)dout; a.lddo = lddo;
-    a.dot = (const uint16_t*)dot; a.delta = delta;
-    a.dq = (uint16_t*)dq; a.dk = (uint16_t*)dk; a.dv = (uint16_t*)dv;
-    a.lddq = lddq; a.lddk = lddk; a.lddv = lddv;
-    a.rcos = (const uint16_t*)rope_cos; a.rsin = (const uint16_t*)rope_sin;
-    rope_done = true;
-    a.B = (int)B; a.S = (int)S; a.H = (int)H; a.KV = (int)KV; a.scale = scale;
-    const unsigned grid_kv = (unsigned)(lz_cdiv(S, 128) * B * KV);
-    const unsigned grid_q = (unsigned)(lz_cdiv(S, 128) * B * H);
-    if (hd == 128) {
-      attn_bwd_dkdv_kernel<128><<<grid_kv, 256, 0, s>>>(a);
-      attn_bwd_dq_kernel<128><<<grid_q, 256, 0, s>>>(a);
-    } else {
-      attn_bwd_dkdv_kernel<64><<<grid_kv, 256, 0, s>>>(a);
-      attn_bwd_dq_kernel<64><<<grid_q, 256, 0, s>>>(a);
-    }
-    return lz_check_launch("lz_attn_bwd");
-  }
+  LZ_REQUIRE(!(mfma && dtype == LZ_BF16 && S % 64) || (qt && kt && dot),
+             "lz_attn_bwd: this shape takes transposed Q, K and dO buffers");
+  if (mfma && (dtype == LZ_BF16 || S % 64 == 0))
+    return tiles_bwd(q, ldq, k, ldk, v, ldv, dout, lddo, lse, delta, dq, lddq, dk, lddk, dv, lddv, B, S, H, KV, hd,
+                     scale, rope_cos, rope_sin, dtype, s, rope_done, o, ldo, delta_w);
+  LzWaveArgs w = wave_fwd_args(q, ldq, k, ldk, v, ldv, nullptr, 0, const_cast<float*>(lse), B, S, H, KV, scale);
+  wave_bwd_args(w, dout, lddo, delta, dq, lddq, dk, lddk, dv, lddv);
+  if (lz_attn_wave_ok(w, dtype, hd, true)) return lz_attn_wave_bwd(w, dtype, hd, kWaveSplit, s);
   const unsigned grid_q = (unsigned)lz_cdiv(B * H * S, 4);
   const unsigned grid_kv = (unsigned)lz_cdiv(B * KV * S, 4);
   if (dtype == LZ_BF16) {
@@ -2147,13 +1646,8 @@ int attn_bwd_impl(const void* q, int64_t ldq, const void* k, int64_t ldk, const 
 
 namespace {
 
-template <typename T>
-int general_args(GenArgs<T>& a, const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
-                 const void* mask, int mask_kind, const int64_t* mstride, float dropout_p, uint64_t seed, int64_t B,
-                 int64_t S, int64_t H, int64_t KV, int64_t hd, float scale) {
-  a.q = (const T*)q; a.k = (const T*)k; a.v = (const T*)v;
-  a.ldq = ldq; a.ldk = ldk; a.ldv = ldv;
-  a.B = (int)B; a.S = (int)S; a.H = (int)H; a.KV = (int)KV; a.hd = (int)hd; a.scale = scale;
+template <class A>
+void general_args(A& a, const void* mask, int mask_kind, const int64_t* mstride, float dropout_p, uint64_t seed) {
   a.mask = mask; a.mask_kind = mask_kind;
   if (mask_kind) {
     a.msb = mstride[0]; a.msh = mstride[1]; a.msq = mstride[2]; a.msk = mstride[3];
@@ -2161,7 +1655,16 @@ int general_args(GenArgs<T>& a, const void* q, int64_t ldq, const void* k, int64
   a.drop_thresh = (uint32_t)std::min(std::ceil((double)dropout_p * 16777216.0), 16777216.0);
   a.drop_scale = dropout_p < 1.f ? 1.0f / (1.0f - dropout_p) : 0.f;
   a.drop_seed = seed;
-  return LZ_OK;
+}
+
+template <typename T>
+void general_args(GenArgs<T>& a, const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
+                 const void* mask, int mask_kind, const int64_t* mstride, float dropout_p, uint64_t seed, int64_t B,
+                 int64_t S, int64_t H, int64_t KV, int64_t hd, float scale) {
+  a.q = (const T*)q; a.k = (const T*)k; a.v = (const T*)v;
+  a.ldq = ldq; a.ldk = ldk; a.ldv = ldv;
+  a.B = (int)B; a.S = (int)S; a.H = (int)H; a.KV = (int)KV; a.hd = (int)hd; a.scale = scale;
+  general_args(a, mask, mask_kind, mstride, dropout_p, seed);
 }
 
 int check_general(const void* mask, int mask_kind, const int64_t* mstride, float dropout_p) {
@@ -2177,8 +1680,9 @@ int check_general(const void* mask, int mask_kind, const int64_t* mstride, float
 
 }  // namespace
 
-// Attention on the one-wave-per-row kernels with the options the tile paths
-// do not take (model/llama.py:109-117, F.scaled_dot_product_attention):
+// Attention with the options the tile paths do not take, on the wave-private
+// kernels (attn_wave.hip; other head dims and unaligned rows: one wave per
+// row) (model/llama.py:109-117, F.scaled_dot_product_attention):
 //   - an explicit mask in place of the causal one (attn_mask with
 //     is_causal=False): mask_kind 1 = bool bytes (nonzero: the key takes
 //     part), 2 = fp32, 3 = bf16, 4 = fp16 (added to the scaled scores); mstride = its
@@ -2188,7 +1692,7 @@ int check_general(const void* mask, int mask_kind, const int64_t* mstride, float
 //   - attention dropout (dropout_p): each probability kept with scale
 //     1/(1-p) by element ((b*H + h)*S + s)*S + kv of seed's stream (the
 //     stream lz_dropout uses), the normaliser summing them before dropout.
-// Any head dim up to 256, bf16 or fp32.
+// Any head dim up to 256, any dtype.
 LZ_EXPORT int lz_attn_fwd_general(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
                                   const void* mask, int mask_kind, const int64_t* mstride, float dropout_p,
                                   uint64_t seed, void* o, int64_t ldo, float* lse, int64_t B, int64_t S, int64_t H,
@@ -2199,6 +1703,11 @@ LZ_EXPORT int lz_attn_fwd_general(const void* q, int64_t ldq, const void* k, int
   if (rc) return rc;
   LZ_REQUIRE(q && k && v && o && lse, "lz_attn_fwd_general: null pointer");
   hipStream_t s = lz_stream(stream);
+  LzWaveArgs w = wave_fwd_args(q, ldq, k, ldk, v, ldv, o, ldo, lse, B, S, H, KV, scale);
+  if (lz_attn_wave_ok(w, dtype, hd, false)) {
+    general_args(w, mask, mask_kind, mstride, dropout_p, seed);
+    return lz_attn_wave_pass(w, dtype, hd, kWaveGeneral, kWaveFwd, s);
+  }
   const unsigned grid = (unsigned)lz_cdiv(B * H * S, 4);
   if (dtype == LZ_BF16) {
     GenArgs<uint16_t> a{};
@@ -2235,6 +1744,12 @@ LZ_EXPORT int lz_attn_bwd_general(const void* q, int64_t ldq, const void* k, int
   if (rc) return rc;
   LZ_REQUIRE(q && k && v && dout && lse && delta && dq && dk && dv, "lz_attn_bwd_general: null pointer");
   hipStream_t s = lz_stream(stream);
+  LzWaveArgs w = wave_fwd_args(q, ldq, k, ldk, v, ldv, nullptr, 0, const_cast<float*>(lse), B, S, H, KV, scale);
+  wave_bwd_args(w, dout, lddo, delta, dq, lddq, dk, lddk, dv, lddv);
+  if (lz_attn_wave_ok(w, dtype, hd, true)) {
+    general_args(w, mask, mask_kind, mstride, dropout_p, seed);
+    return lz_attn_wave_bwd(w, dtype, hd, kWaveGeneral, s);
+  }
   const unsigned grid_q = (unsigned)lz_cdiv(B * H * S, 4);
   const unsigned grid_kv = (unsigned)lz_cdiv(B * KV * S, 4);
   if (dtype == LZ_BF16) {
@@ -2262,4 +1777,52 @@ LZ_EXPORT int lz_attn_bwd_general(const void* q, int64_t ldq, const void* k, int
     return lz_set_error(LZ_EINVAL, "lz_attn_bwd_general: bad dtype %d", dtype);
   }
   return lz_check_launch("lz_attn_bwd_general");
+}
+
+// Whether lz_attn_fwd_direct / lz_attn_bwd_direct take these shapes: head dim
+// 32, 64 or 128, row strides of whole 16-byte pieces.
+LZ_EXPORT int lz_attn_direct(int dtype, int64_t hd, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo) {
+  const int64_t rd = dtype == LZ_F32 ? 4 : 8;
+  return (dtype == LZ_BF16 || dtype == LZ_F16 || dtype == LZ_F32) && (hd == 32 || hd == 64 || hd == 128) &&
+         ldq % rd == 0 && ldk % rd == 0 && ldv % rd == 0 && ldo % rd == 0;
+}
+
+// Causal attention of any sequence length that reads q, k and v (and o and
+// dout in the backward) as they are stored: no transposed copies and no
+// separate delta pass (the backward writes delta [B, H, S], which it forms
+// from o and dout).  Shapes outside lz_attn_direct and unaligned pointers
+// are refused.
+LZ_EXPORT int lz_attn_fwd_direct(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
+                                 void* o, int64_t ldo, float* lse, int64_t B, int64_t S, int64_t H, int64_t KV,
+                                 int64_t hd, float scale, int dtype, void* stream) {
+  int rc = check_shape(B, S, H, KV, hd);
+  if (rc) return rc;
+  LZ_REQUIRE(q && k && v && o && lse, "lz_attn_fwd_direct: null pointer");
+  const LzWaveArgs w = wave_fwd_args(q, ldq, k, ldk, v, ldv, o, ldo, lse, B, S, H, KV, scale);
+  LZ_REQUIRE(lz_attn_direct(dtype, hd, ldq, ldk, ldv, ldo) && lz_attn_wave_ok(w, dtype, hd, false),
+             "lz_attn_fwd_direct: unsupported head dim, dtype or alignment");
+  if (dtype == LZ_BF16 && mfma_ok(dtype, hd, ldq, ldk, ldv, ldo, q, k, v, o))
+    return tiles_fwd(q, ldq, k, ldk, v, ldv, o, ldo, lse, B, S, H, KV, hd, scale, dtype, lz_stream(stream));
+  return lz_attn_wave_pass(w, dtype, hd, kWaveSplit, kWaveFwd, lz_stream(stream));
+}
+
+LZ_EXPORT int lz_attn_bwd_direct(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
+                                 const void* o, int64_t ldo, const void* dout, int64_t lddo, const float* lse,
+                                 float* delta, void* dq, int64_t lddq, void* dk, int64_t lddk, void* dv, int64_t lddv,
+                                 int64_t B, int64_t S, int64_t H, int64_t KV, int64_t hd, float scale, int dtype,
+                                 void* stream) {
+  int rc = check_shape(B, S, H, KV, hd);
+  if (rc) return rc;
+  LZ_REQUIRE(q && k && v && o && dout && lse && delta && dq && dk && dv, "lz_attn_bwd_direct: null pointer");
+  LzWaveArgs w = wave_fwd_args(q, ldq, k, ldk, v, ldv, const_cast<void*>(o), ldo, const_cast<float*>(lse), B, S, H, KV,
+                               scale);
+  wave_bwd_args(w, dout, lddo, nullptr, dq, lddq, dk, lddk, dv, lddv);
+  w.delta_w = delta;
+  LZ_REQUIRE(lz_attn_direct(dtype, hd, ldq, ldk, ldv, ldo) && lz_attn_wave_ok(w, dtype, hd, true),
+             "lz_attn_bwd_direct: unsupported head dim, dtype or alignment");
+  bool rope_done = false;
+  if (dtype == LZ_BF16 && mfma_ok(dtype, hd, ldq, ldk, ldv, lddo, q, k, v, dout))
+    return tiles_bwd(q, ldq, k, ldk, v, ldv, dout, lddo, lse, nullptr, dq, lddq, dk, lddk, dv, lddv, B, S, H, KV, hd,
+                     scale, nullptr, nullptr, dtype, lz_stream(stream), rope_done, o, ldo, delta);
+  return lz_attn_wave_bwd(w, dtype, hd, kWaveSplit, lz_stream(stream));
 }

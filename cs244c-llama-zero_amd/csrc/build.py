@@ -32,6 +32,7 @@ SOURCES = [
     "gemm.hip",
     "gemm_f32.hip",
     "attn.hip",
+    "attn_wave.hip",
 ]
 
 COMMON_FLAGS = [

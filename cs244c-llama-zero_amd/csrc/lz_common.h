@@ -109,6 +109,13 @@ __device__ __forceinline__ void lz_dma16_first(lz_v4i rsrc, uint32_t voff, uint3
                :: "v"(voff), "s"(rsrc), "s"(soff), "{m0}"(m0) : "memory");
 }
 
+// Direct-to-LDS copy of 4 bytes per lane (lane l's to dst + 4*l), with the
+// wait states of lz_dma16_first: for rows without 16-byte alignment.
+__device__ __forceinline__ void lz_dma4_first(lz_v4i rsrc, uint32_t voff, void* dst) {
+  const uint32_t m0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)dst;
+  asm volatile("s_nop 4\n\tbuffer_load_dword %0, %1, 0 offen lds" :: "v"(voff), "s"(rsrc), "{m0}"(m0) : "memory");
+}
+
 // 16-byte store with the nontemporal hint (global_store_dwordx4 ... nt): for
 // outputs a kernel writes once and does not read back, so that they do not
 // displace the operand rows the rest of the grid is still reading from L2.

@@ -111,6 +111,18 @@ SIGNATURES = {
             _i64, _i64, _i64, _i64, _i64, _f32, _vp, _vp, _i32, _vp,
         ],
     ),
+    "lz_attn_direct": (_i32, [_i32, _i64, _i64, _i64, _i64, _i64]),
+    "lz_attn_fwd_direct": (
+        _i32,
+        [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _f32, _i32, _vp],
+    ),
+    "lz_attn_bwd_direct": (
+        _i32,
+        [
+            _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _i64,
+            _i64, _i64, _i64, _i64, _i64, _f32, _i32, _vp,
+        ],
+    ),
     "lz_dropout": (_i32, [_vp, _vp, _i64, _f32, _u64, _i32, _vp]),
     "lz_dropout_mask": (_i32, [_vp, _i64, _f32, _u64, _vp]),
     "lz_attn_bwd": (

@@ -360,7 +360,7 @@ class AttnProjFn(Function):
     weights Wq [H*hd, d], Wk/Wv [KV*hd, d]; returns the attention output
     [B, S, H*hd] that o_proj consumes.  mask: SDPA's attn_mask in place of
     the causal mask; dropout_p > 0: attention dropout with the stream key
-    `seed` (both on the one-wave-per-row kernels)."""
+    `seed` (both through ops.attn_fwd_general)."""
 
     @staticmethod
     def forward(ctx, h, wq, wk, wv, cos, sin, n_heads: int, n_kv: int, scale: float, mask=None,
@@ -384,10 +384,11 @@ class AttnProjFn(Function):
         if general:
             o, lse = ops.attn_fwd_general(q2, k2, v2, B, S, H, KV, hd, scale, mask, dropout_p, seed)
         else:
-            vt = None
-            if ops.attn_path(qkv.dtype, S, hd, ld, ld, ld, H * hd) == 1:
-                vt = ops.transpose_heads(qkv, B, S, KV, hd, col0=(H + KV) * hd)
-            o, lse = ops.attn_fwd(q2, k2, v2, B, S, H, KV, hd, scale, vt)
+            tiles = ops.attn_path(qkv.dtype, S, hd, ld, ld, ld, H * hd) == 2
+            if not tiles and ops.attn_direct(q2, k2, v2, hd):
+                o, lse = ops.attn_fwd_direct(q2, k2, v2, B, S, H, KV, hd, scale)
+            else:
+                o, lse = ops.attn_fwd(q2, k2, v2, B, S, H, KV, hd, scale, None)
         ctx.save_for_backward(h2, wq, wk, wv, qkv, o, lse, cos, sin)
         ctx.mask = mask
         ctx.general = (general, dropout_p, seed)
@@ -408,12 +409,11 @@ class AttnProjFn(Function):
             ops.attn_bwd_general(q2, k2, v2, o, do2, lse, B, S, H, KV, hd, scale, dq2, dk2, dv2, ctx.mask,
                                  dropout_p, seed)
         else:
-            qt = kt = dot = None
-            if ops.attn_path(qkv.dtype, S, hd, ld, ld, ld, do2.stride(0)) == 1:
-                qt = ops.transpose_heads(qkv, B, S, H, hd, col0=0)
-                kt = ops.transpose_heads(qkv, B, S, KV, hd, col0=H * hd)
-                dot = ops.transpose_heads(do2, B, S, H, hd, col0=0)
-            ops.attn_bwd(q2, k2, v2, o, do2, lse, B, S, H, KV, hd, scale, dq2, dk2, dv2, qt=qt, kt=kt, dot=dot)
+            tiles = ops.attn_path(qkv.dtype, S, hd, ld, ld, ld, do2.stride(0)) == 2
+            if not tiles and ops.attn_direct(q2, k2, v2, hd, o, do2):
+                ops.attn_bwd_direct(q2, k2, v2, o, do2, lse, B, S, H, KV, hd, scale, dq2, dk2, dv2)
+            else:
+                ops.attn_bwd(q2, k2, v2, o, do2, lse, B, S, H, KV, hd, scale, dq2, dk2, dv2)
         # RoPE's backward as its own pass over dq|dk: attn_bwd(rope=...) can
         # fold it into the dQ/dK stores, but in the MFMA output layout each
         # lane's table reads are 8-byte pieces of 32 different rows, which

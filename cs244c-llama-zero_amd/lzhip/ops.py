@@ -971,8 +971,10 @@ def ce_bwd(logits2: torch.Tensor, labels: torch.Tensor, seq: int, lse: torch.Ten
 
 
 def attn_path(dtype: torch.dtype, S: int, hd: int, ldq: int, ldk: int, ldv: int, ldo: int) -> int:
-    """2: MFMA on LDS tiles (no transposed operands), 1: MFMA with transposed
-    operand buffers (V^T forward; Q^T, K^T, dO^T backward), 0: generic."""
+    """What attn_fwd/attn_bwd take: 2: MFMA on LDS tiles, 1: the same at other
+    lengths, where they ask for transposed operand buffers (V^T forward; Q^T,
+    K^T, dO^T backward) and attn_fwd_direct/attn_bwd_direct do not, 0: the
+    rest."""
     if dtype not in _DTYPES:
         return 0
     return int(_lib.load().lz_attn_path(_DTYPES[dtype], S, hd, ldq, ldk, ldv, ldo))
@@ -991,6 +993,39 @@ def attn_fwd(q2: torch.Tensor, k2: torch.Tensor, v2: torch.Tensor, B: int, S: in
     return o, lse
 
 
+def attn_direct(q2: torch.Tensor, k2: torch.Tensor, v2: torch.Tensor, hd: int, *rows: torch.Tensor) -> bool:
+    """Whether attn_fwd_direct (rows: none) or attn_bwd_direct (rows: o, do)
+    takes these row views: head dim 32, 64 or 128, 16-byte aligned rows."""
+    if q2.dtype not in _DTYPES:
+        return False
+    strides = [_row_stride(t) for t in (q2, k2, v2)]
+    lib = _lib.load()
+    return (all(t.data_ptr() % 16 == 0 for t in (q2, k2, v2, *rows))
+            and all(lib.lz_attn_direct(_DTYPES[q2.dtype], hd, *strides, _row_stride(t)) for t in (rows or (q2,))))
+
+
+def attn_fwd_direct(q2: torch.Tensor, k2: torch.Tensor, v2: torch.Tensor, B: int, S: int, H: int, KV: int, hd: int,
+                    scale: float) -> Tuple[torch.Tensor, torch.Tensor]:
+    """attn_fwd for any sequence length from q/k/v as stored (attn_direct)."""
+    require_gpu(q2, k2, v2)
+    o = torch.empty((B * S, H * hd), dtype=q2.dtype, device=q2.device)
+    lse = torch.empty((B, H, S), dtype=torch.float32, device=q2.device)
+    _lib.call("lz_attn_fwd_direct", q2.data_ptr(), _row_stride(q2), k2.data_ptr(), _row_stride(k2), v2.data_ptr(),
+              _row_stride(v2), o.data_ptr(), H * hd, lse.data_ptr(), B, S, H, KV, hd, float(scale), dtype_code(q2),
+              stream_ptr(q2.device))
+    return o, lse
+
+
+def attn_bwd_direct(q2, k2, v2, o2, do2, lse, B, S, H, KV, hd, scale, dq2, dk2, dv2) -> None:
+    """Backward of attn_fwd_direct (delta is formed inside)."""
+    require_gpu(q2, k2, v2, o2, do2, lse, dq2, dk2, dv2)
+    delta = torch.empty((B, H, S), dtype=torch.float32, device=q2.device)
+    _lib.call("lz_attn_bwd_direct", q2.data_ptr(), _row_stride(q2), k2.data_ptr(), _row_stride(k2), v2.data_ptr(),
+              _row_stride(v2), o2.data_ptr(), _row_stride(o2), do2.data_ptr(), _row_stride(do2), lse.data_ptr(),
+              delta.data_ptr(), dq2.data_ptr(), _row_stride(dq2), dk2.data_ptr(), _row_stride(dk2), dv2.data_ptr(),
+              _row_stride(dv2), B, S, H, KV, hd, float(scale), dtype_code(q2), stream_ptr(q2.device))
+
+
 def _attn_mask_args(mask: torch.Tensor, B: int, H: int, S: int):
     """(kind, strides array) of an attention mask broadcastable to [B, H, S, S]
     (bool: True keeps the score; fp32/bf16: added to it)."""
@@ -1007,7 +1042,8 @@ def _attn_mask_args(mask: torch.Tensor, B: int, H: int, S: int):
 
 def attn_fwd_general(q2, k2, v2, B: int, S: int, H: int, KV: int, hd: int, scale: float,
                      mask: Optional[torch.Tensor] = None, dropout_p: float = 0.0, seed: int = 0):
-    """attn_fwd on the one-wave-per-row kernels, with an explicit mask in
+    """attn_fwd on the wave-private kernels (other head dims: one wave per
+    row), with an explicit mask in
     place of the causal one (mask=None: causal) and/or attention dropout
     (dropout_p with seed, see dropout_seed); returns o, lse."""
     require_gpu(q2, k2, v2)

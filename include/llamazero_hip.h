@@ -298,11 +298,13 @@ int lz_gemm_swiglu_bwd(const void* dy, int64_t lddy, const void* w, int64_t ldw,
                        void* dgu, int64_t lddgu, int64_t M, int64_t F, int64_t K, void* stream);
 
 /* Causal GQA flash attention (model/llama.py:88-117: repeat_kv +
- * F.scaled_dot_product_attention(is_causal=True)).  lz_attn_path reports the
- * path lz_attn_fwd/bwd take: 2 = MFMA on LDS tiles (bf16 or fp16, hd 64 or 128, S a
- * multiple of 64; the transposed-operand arguments may be NULL), 1 = MFMA
- * with the transposed operand buffers (vt for the forward; qt, kt, dot for the
- * backward, each [B, heads, hd, S]), 0 = generic. */
+ * F.scaled_dot_product_attention(is_causal=True)).  lz_attn_path reports what
+ * lz_attn_fwd/bwd take: 2 = MFMA on LDS tiles (bf16 or fp16, hd 64 or 128, S a
+ * multiple of 64; the transposed-operand arguments may be NULL), 1 = bf16 at
+ * other lengths: vt (forward) and qt, kt, dot (backward, each [B, heads, hd,
+ * S]) are required though no kernel reads them any more (the direct entry
+ * points below take the same shapes without them), 0 = the rest (hd 32 and
+ * fp32: wave-private MFMA kernels; other head dims: generic). */
 int lz_attn_path(int dtype, int64_t S, int64_t hd, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo);
 int lz_attn_fwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, const void* vt,
                 void* o, int64_t ldo, float* lse, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t hd, float scale,
@@ -313,8 +315,7 @@ int lz_attn_delta(const void* o, int64_t ldo, const void* dout, int64_t lddo, fl
  * are returned as the gradients of q and k before RoPE (model/llama.py:35-39
  * backward), folded into the bf16 MFMA kernels' stores or, on the other
  * paths, applied by lz_rope afterwards. */
-/* Attention on the one-wave-per-row kernels with the options the MFMA tile
- * paths do not take (model/llama.py:105-117, F.scaled_dot_product_attention):
+/* Attention with the options the MFMA tile paths do not take (model/llama.py:105-117, F.scaled_dot_product_attention):
  *  - an explicit mask in place of the causal one (attn_mask with
  *    is_causal=False): mask_kind 1 = bool bytes (nonzero: the key takes
  *    part), 2 = fp32, 3 = bf16, 4 = fp16 (added to the scaled scores); mstride = 4
@@ -351,6 +352,20 @@ int lz_attn_bwd_with_o(const void* q, int64_t ldq, const void* k, int64_t ldk, c
                        void* dq, int64_t lddq, void* dk, int64_t lddk, void* dv, int64_t lddv, int64_t B, int64_t S,
                        int64_t H, int64_t KV, int64_t hd, float scale, const void* rope_cos, const void* rope_sin,
                        int dtype, void* stream);
+
+/* Causal attention of any sequence length straight from q, k, v (o, dout) rows
+ * as stored: no transposed copies, no separate delta pass (the backward
+ * forms delta [B, H, S], an output, from o and dout).  Takes what
+ * lz_attn_direct reports (hd 32, 64 or 128; row strides of whole 16-byte
+ * pieces) with 16-byte aligned pointers; others are refused. */
+int lz_attn_direct(int dtype, int64_t hd, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo);
+int lz_attn_fwd_direct(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, void* o,
+                       int64_t ldo, float* lse, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t hd, float scale,
+                       int dtype, void* stream);
+int lz_attn_bwd_direct(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
+                       const void* o, int64_t ldo, const void* dout, int64_t lddo, const float* lse, float* delta,
+                       void* dq, int64_t lddq, void* dk, int64_t lddk, void* dv, int64_t lddv, int64_t B, int64_t S,
+                       int64_t H, int64_t KV, int64_t hd, float scale, int dtype, void* stream);
 
 /* ---- dropout (model/llama.py:142,146 on the MLP's gated activations and
  * :175,213 on the token embeddings: nn.Dropout in training mode) ----

@@ -1166,3 +1166,83 @@ def test_copy2d_exact(dtype):
     want = torch.zeros(16, 64, dtype=dtype)
     want[:, 4:36] = src.cpu()[:, 4:36]
     assert torch.equal(dst.cpu(), want)
+
+
+@pytest.mark.parametrize("hd", [32, 64, 128])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B,S,H,KV,kind", [(1, 1, 2, 1, None), (2, 31, 4, 2, None), (1, 33, 5, 1, None),
+                                           (1, 65, 2, 2, None), (1, 321, 4, 1, None), (1, 600, 8, 8, None),
+                                           (2, 63, 4, 2, "bool"), (2, 130, 4, 1, "bool"), (1, 97, 2, 2, "lowest"),
+                                           (1, 96, 4, 2, "strided"), (1, 40, 2, 1, "dropout")])
+def test_attention_wave_private_kernels(B, S, H, KV, kind, hd, dtype):
+    """The wave-private kernels (and the ragged tile kernels: S 600 of bf16
+    heads of 64 and 128) at the edges of their 32- and 64-row tiles, against
+    float64: causal, bool masks with a query that sees nothing (NaN there and
+    only there) and keys nobody sees (their V may hold inf), additive masks
+    of the type's lowest value and of arbitrary strides, and dropout.
+    Tolerances: one rounding of the output type (bf16 2^-9, fp16 2^-12 per
+    value) of intermediate P or O, fp32 sums 1e-5, as the tests above."""
+    g = _seed(B * S + hd + len(kind or ""))
+    ld = (H + 2 * KV) * hd
+    qkv = torch.randn(B * S, ld, generator=g).to(dtype)
+    d = qkv.to(DEV)
+    q2, k2, v2 = d[:, : H * hd], d[:, H * hd : (H + KV) * hd], d[:, (H + KV) * hd :]
+    do = torch.randn(B * S, H * hd, generator=g).to(dtype)
+    scale = hd**-0.5
+    mask = mdev = keep = None
+    p = key = 0
+    if kind == "bool":
+        mask = ~torch.triu(torch.ones(S, S, dtype=torch.bool), 1).repeat(B, 1, 1, 1)
+        mask[:, :, :, S - 35 :] = False  # keys nobody sees
+        mask[0, 0, 5, :] = False  # a query that sees nothing
+        d[S - 1, (H + KV) * hd :] = float("inf")
+    elif kind == "lowest":
+        low = torch.finfo(dtype).min
+        mask = torch.zeros(B, 1, S, S, dtype=dtype).masked_fill(torch.triu(torch.ones(S, S, dtype=torch.bool), 1), low)
+        mask[0, 0, 7, :] = low  # every key lowest: a plain mean over them; its lse
+        do[7] = 0               # (lowest + log S) keeps no log S in fp32, so no gradient is asked of it
+    elif kind == "strided":
+        mask = torch.randn(B, S, H, S, generator=g).permute(0, 2, 3, 1)
+    if mask is not None:
+        mdev = mask.to(DEV) if kind != "strided" else mask.permute(0, 3, 1, 2).contiguous().to(DEV).permute(0, 2, 3, 1)
+    if kind == "dropout":
+        p, key = 0.25, ops.dropout_key(7, S)
+        keep = ops.dropout_mask(B * H * S * S, p, key, DEV).cpu().view(B, H, S, S)
+    dqkv = torch.zeros_like(d)
+    grads = dqkv[:, : H * hd], dqkv[:, H * hd : (H + KV) * hd], dqkv[:, (H + KV) * hd :]
+    if kind is None:
+        o, lse = ops.attn_fwd_direct(q2, k2, v2, B, S, H, KV, hd, scale)
+        ops.attn_bwd_direct(q2, k2, v2, o, do.to(DEV), lse, B, S, H, KV, hd, scale, *grads)
+    else:
+        o, lse = ops.attn_fwd_general(q2, k2, v2, B, S, H, KV, hd, scale, mdev, p, key)
+        if kind == "bool":
+            d[S - 1, (H + KV) * hd :] = qkv[S - 1, (H + KV) * hd :].to(DEV)
+        ops.attn_bwd_general(q2, k2, v2, o, do.to(DEV), lse, B, S, H, KV, hd, scale, *grads, mdev, p, key)
+
+    def heads(t, n):
+        return t.double().view(B, S, n, hd).transpose(1, 2)
+
+    qr, kr, vr = (heads(t, n).requires_grad_(True) for t, n in (
+        (qkv[:, : H * hd], H), (qkv[:, H * hd : (H + KV) * hd], KV), (qkv[:, (H + KV) * hd :], KV)))
+    mref = mask if mask is None or mask.dtype == torch.bool else mask.double()
+    oref = R.causal_gqa_attention(qr, kr, vr, scale, attn_mask=mref, dropout_keep=keep, dropout_p=p)
+    otol, gtol = {torch.bfloat16: (1e-2, 2e-2), torch.float16: (2e-3, 5e-3), torch.float32: (1e-5, 1e-5)}[dtype]
+    got = heads(o.cpu(), H)
+    if kind == "bool":
+        assert bool(got[0, :, 5].isnan().all()) and bool(torch.isneginf(lse[0, :, 5]).all())
+        assert bool(heads(grads[0].cpu(), H)[0, :, 5].isnan().all())
+        assert bool(heads(grads[1].cpu(), KV)[0].isnan().all())  # that query's NaN reaches every key of its batch
+        fine = torch.ones(B, S, dtype=torch.bool)
+        fine[0, 5] = False
+        sel = lambda t: t.transpose(1, 2)[fine]  # noqa: E731
+        assert _rel_err(sel(got), sel(oref)) < otol
+        if B > 1:  # the other sequences' gradients are untouched by it
+            (oref[1:] * heads(do, H)[1:]).sum().backward()
+            for got_g, want in zip(grads, (qr.grad, kr.grad, vr.grad)):
+                assert _rel_err(heads(got_g.cpu(), want.shape[1])[1:], want[1:]) < gtol
+        return
+    assert _rel_err(got, oref) < otol
+    oref.backward(heads(do, H))
+    for got_g, want in zip(grads[:2], (qr.grad, kr.grad)):
+        assert _grad_err(heads(got_g.cpu(), want.shape[1]), want, vr.grad) < gtol
+    assert _rel_err(heads(grads[2].cpu(), KV), vr.grad) < gtol
