@@ -30,6 +30,7 @@ SOURCES = [
     "ce.hip",
     "transpose.hip",
     "gemm.hip",
+    "gemm_pipe.hip",
     "gemm_f32.hip",
     "attn.hip",
     "attn_wave.hip",

@@ -665,9 +665,11 @@ def gemm_kernel_name(key) -> str:
         name = f"gemm_dma_kernel<FmtBF16, 2, 4, {tf(ak)}, {tf(bk)}, 64, 2>"
     elif cfg == 6:
         name = f"gemm_dma_n192_kernel<FmtBF16, {tf(bk)}>"
+    elif cfg >= 7:
+        bm, bn, wn, stages = {7: (128, 128, 4, 2), 8: (64, 128, 4, 3), 9: (64, 64, 2, 3)}[cfg]
+        name = f"gemm_pipe_kernel<FmtBF16, {bm}, {bn}, 2, {wn}, {tf(ak)}, {tf(bk)}, {stages}>"
     else:
-        bm, wn = (128, 2) if cfg == 2 else (256, 4 if cfg == 0 else 2)
-        name = f"gemm_kernel<FmtBF16, {bm}, {bm}, 2, {wn}, {tf(ak)}, {tf(bk)}>"
+        name = f"gemm_kernel<FmtBF16, 256, 256, 2, {4 if cfg == 0 else 2}, {tf(ak)}, {tf(bk)}>"
     return name + (f" split-K x{splits} (+ splitk_reduce_kernel)" if splits > 1 else "")
 
 

@@ -1246,3 +1246,65 @@ def test_attention_wave_private_kernels(B, S, H, KV, kind, hd, dtype):
     for got_g, want in zip(grads[:2], (qr.grad, kr.grad)):
         assert _grad_err(heads(got_g.cpu(), want.shape[1]), want, vr.grad) < gtol
     assert _rel_err(heads(grads[2].cpu(), KV), vr.grad) < gtol
+
+
+@pytest.mark.parametrize("ak,bk", [(True, True), (True, False), (False, False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(8, 8, 8), (64, 128, 64), (72, 200, 56), (200, 72, 328), (320, 448, 1000),
+                                   (776, 768, 2056), (1152, 1152, 1024), (136, 64, 4096), (2048, 1280, 136)])
+def test_gemm_small_tiles(M, N, K, dtype, ak, bk):
+    """The small-tile kernels (plan codes 7-9) on edge tiles, K tails, one and
+    several K slices and every epilogue, against float64.  The operands are
+    views whose padding holds NaN: nothing outside them may be read into a
+    result.  Tolerances as test_gemm_n192_tiles."""
+    lib = _lib.load()
+    code = int(lib.lz_gemm_plan(M, N, K, int(ak), int(bk)))
+    assert code // 64 in (7, 8, 9)
+    g = _seed(M + 7 * N + K + 2 * ak + bk)
+    a = torch.randn(M, K, generator=g).to(dtype)
+    b = torch.randn(N, K, generator=g).to(dtype)
+    ref = a.double() @ b.double().t()
+
+    def operand(t, kmajor):
+        t = t if kmajor else t.t()
+        buf = torch.full((t.shape[0], t.shape[1] + 8), float("nan"), dtype=dtype)
+        buf[:, : t.shape[1]] = t
+        return buf.to(DEV)[:, : t.shape[1]]
+
+    A, B = operand(a, ak), operand(b, bk)
+    tol = 1e-5 * math.sqrt(K) * float(a.float().abs().max() * b.float().abs().max()) * 4
+    eps = 2 ** -8 if dtype == torch.bfloat16 else 2 ** -11
+    c32 = ops.gemm(A, B, ak, bk, out_dtype=torch.float32).cpu()
+    assert float((c32.double() - ref).abs().max()) <= tol
+    c16 = ops.gemm(A, B, ak, bk).cpu()
+    assert torch.equal(c16, c32.to(dtype))
+    r = torch.randn(M, N, generator=g).to(dtype)
+    assert torch.equal(ops.gemm(A, B, ak, bk, residual=r.to(DEV)).cpu(), (c16.float() + r.float()).to(dtype))
+    h0 = torch.randn(M, N, generator=g).to(dtype)
+    acc16 = h0.to(DEV)
+    ops.gemm(A, B, ak, bk, out=acc16, alpha=0.5, beta=1.0)
+    want = 0.5 * ref + h0.double()
+    assert bool(((acc16.cpu().double() - want).abs() <= eps * want.abs() + 0.5 * tol + 1e-6).all())
+    wide = torch.zeros(M, N + 3, dtype=torch.float32, device=DEV)  # rows without 16-byte alignment
+    ops.gemm(A, B, ak, bk, out=wide[:, :N])
+    assert torch.equal(wide[:, :N].cpu(), c32) and float(wide[:, N:].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(4096, 4096, 2001), (2048, 5632, 8197), (4104, 4088, 1087)])
+def test_gemm_weight_gradient_k_tail(M, N, K, dtype):
+    """dy^T . x over a token count that is not a multiple of 64 on the
+    direct-to-LDS kernel, split and unsplit, with NaN in the rows after the
+    last one: against float64 within the fp32 sums' tolerance."""
+    lib = _lib.load()
+    assert int(lib.lz_gemm_plan(M, N, K, 0, 0)) // 64 == 5
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    a = torch.full((K + 64, M), float("nan"), device=DEV, dtype=dtype)
+    b = torch.full((K + 64, N), float("nan"), device=DEV, dtype=dtype)
+    a[:K] = torch.randn(K, M, device=DEV, generator=g).to(dtype)
+    b[:K] = torch.randn(K, N, device=DEV, generator=g).to(dtype)
+    c = ops.gemm(a[:K], b[:K], False, False, out_dtype=torch.float32)
+    ref = torch.matmul(a[:K].double().t(), b[:K].double())
+    tol = 1e-5 * math.sqrt(K) * float(a[:K].float().abs().max() * b[:K].float().abs().max()) * 4
+    assert float((c.double() - ref).abs().max()) <= tol
+    assert torch.equal(ops.gemm(a[:K], b[:K], False, False), c.to(dtype))
