@@ -1801,7 +1801,7 @@ LZ_EXPORT int lz_attn_fwd_direct(const void* q, int64_t ldq, const void* k, int6
   const LzWaveArgs w = wave_fwd_args(q, ldq, k, ldk, v, ldv, o, ldo, lse, B, S, H, KV, scale);
   LZ_REQUIRE(lz_attn_direct(dtype, hd, ldq, ldk, ldv, ldo) && lz_attn_wave_ok(w, dtype, hd, false),
              "lz_attn_fwd_direct: unsupported head dim, dtype or alignment");
-  if (dtype == LZ_BF16 && mfma_ok(dtype, hd, ldq, ldk, ldv, ldo, q, k, v, o))
+  if ((dtype == LZ_BF16 || S % 64 == 0) && mfma_ok(dtype, hd, ldq, ldk, ldv, ldo, q, k, v, o))
     return tiles_fwd(q, ldq, k, ldk, v, ldv, o, ldo, lse, B, S, H, KV, hd, scale, dtype, lz_stream(stream));
   return lz_attn_wave_pass(w, dtype, hd, kWaveSplit, kWaveFwd, lz_stream(stream));
 }
@@ -1821,7 +1821,7 @@ LZ_EXPORT int lz_attn_bwd_direct(const void* q, int64_t ldq, const void* k, int6
   LZ_REQUIRE(lz_attn_direct(dtype, hd, ldq, ldk, ldv, ldo) && lz_attn_wave_ok(w, dtype, hd, true),
              "lz_attn_bwd_direct: unsupported head dim, dtype or alignment");
   bool rope_done = false;
-  if (dtype == LZ_BF16 && mfma_ok(dtype, hd, ldq, ldk, ldv, lddo, q, k, v, dout))
+  if ((dtype == LZ_BF16 || S % 64 == 0) && mfma_ok(dtype, hd, ldq, ldk, ldv, lddo, q, k, v, dout))
     return tiles_bwd(q, ldq, k, ldk, v, ldv, dout, lddo, lse, nullptr, dq, lddq, dk, lddk, dv, lddv, B, S, H, KV, hd,
                      scale, nullptr, nullptr, dtype, lz_stream(stream), rope_done, o, ldo, delta);
   return lz_attn_wave_bwd(w, dtype, hd, kWaveSplit, lz_stream(stream));

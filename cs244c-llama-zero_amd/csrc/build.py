@@ -1,7 +1,8 @@
 """Builds libllamazero_hip.so for gfx950 from the .hip sources in this folder.
 
 Each source is compiled to an object under csrc/_build/ (in parallel), then
-linked into ../lzhip/libllamazero_hip.so.  Usage:
+linked into ../lzhip/libllamazero_hip.so; pycall.cpp, the Python entry to it,
+becomes ../lzhip/_pycall.so.  Usage:
 
     python csrc/build.py [--jobs N] [--arch gfx950]
 """
@@ -13,11 +14,13 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
 PKG = HERE.parent
 OUT_LIB = PKG / "lzhip" / "libllamazero_hip.so"
+OUT_CALL = PKG / "lzhip" / "_pycall.so"  # the Python entry to it (pycall.cpp)
 
 SOURCES = [
     "runtime.hip",
@@ -99,7 +102,23 @@ def build(arch: str = "gfx950", jobs: int | None = None, verbose: bool = False) 
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
     os.replace(tmp, OUT_LIB)
+    build_pycall()
     return OUT_LIB
+
+
+def build_pycall() -> Path:
+    """The CPython extension that calls the library (host code only)."""
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("no C++ compiler (g++) for pycall.cpp")
+    tmp = OUT_CALL.with_suffix(".so.tmp")
+    cmd = [cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-I",
+           sysconfig.get_paths()["include"], str(HERE / "pycall.cpp"), "-o", str(tmp)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"pycall.cpp failed:\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, OUT_CALL)
+    return OUT_CALL
 
 
 def main() -> None:

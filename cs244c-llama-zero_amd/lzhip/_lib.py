@@ -1,4 +1,5 @@
-"""ctypes binding of libllamazero_hip.so (declared in include/llamazero_hip.h).
+"""Binding of libllamazero_hip.so (declared in include/llamazero_hip.h): loaded
+with ctypes, its entry points called through _pycall.
 
 The library is loaded after torch so that the process keeps a single HIP
 runtime (torch ships its own libamdhip64.so.7, which the dynamic loader then
@@ -136,6 +137,7 @@ SIGNATURES = {
 
 _lock = threading.Lock()
 _lib = None
+_calls = {}  # entry point name -> its _pycall callable, filled when the library is loaded
 
 
 class HipLibraryError(RuntimeError):
@@ -145,6 +147,8 @@ class HipLibraryError(RuntimeError):
 def load(path: str | os.PathLike | None = None) -> ctypes.CDLL:
     """Loads (once) and returns the library with its signatures applied."""
     global _lib
+    if _lib is not None:  # set once, complete, under the lock
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib
@@ -154,11 +158,18 @@ def load(path: str | os.PathLike | None = None) -> ctypes.CDLL:
                 f"{p} is missing: build it with `python cs244c-llama-zero_amd/csrc/build.py` "
                 "(the HIP kernels are the only compute path)"
             )
+        try:
+            from . import _pycall as pycall
+        except ImportError as e:
+            raise HipLibraryError(f"lzhip/_pycall.so is missing ({e}): build it with "
+                                  "`python cs244c-llama-zero_amd/csrc/build.py`") from e
         lib = ctypes.CDLL(str(p), mode=ctypes.RTLD_GLOBAL)
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
+            if res is not ctypes.c_char_p:
+                _calls[name] = pycall.bind(name, ctypes.cast(fn, _vp).value)
         _lib = lib
         return lib
 
@@ -175,5 +186,15 @@ def check(rc: int, what: str) -> None:
 
 def call(name: str, *args) -> None:
     """Calls an int-returning entry point and raises on a non-zero status."""
-    fn = getattr(load(), name)
-    check(fn(*args), name)
+    if _lib is None:
+        load()
+    rc = _calls[name](*args)
+    if rc != 0:
+        check(rc, name)
+
+
+def query(name: str, *args) -> int:
+    """Calls an entry point that returns a count (a workspace size, a plan)."""
+    if _lib is None:
+        load()
+    return _calls[name](*args)

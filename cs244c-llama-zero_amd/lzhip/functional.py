@@ -178,20 +178,20 @@ def fused_weight(weights: Sequence[torch.Tensor]) -> torch.Tensor:
     w0 = weights[0]
     if len(weights) == 1:
         return w0
-    k = w0.shape[1]
-    n_total = sum(w.shape[0] for w in weights)
-    base = w0.untyped_storage().data_ptr()
-    adjacent = all(
-        w.is_contiguous() and w.dtype == w0.dtype and w.shape[1] == k and w.untyped_storage().data_ptr() == base
-        for w in weights
-    )
+    k, dtype, esz = w0.shape[1], w0.dtype, w0.element_size()
+    n_total = 0
+    expect = w0.data_ptr()
+    adjacent = True
+    for w in weights:
+        n = w.shape[0]
+        n_total += n
+        if adjacent and (w.data_ptr() != expect or w.shape[1] != k or w.dtype != dtype or not w.is_contiguous()):
+            adjacent = False
+        expect += n * k * esz
     if adjacent:
-        expect = w0.data_ptr()
-        for w in weights:
-            if w.data_ptr() != expect:
-                adjacent = False
-                break
-            expect += w.numel() * w.element_size()
+        # one memory range: all of it inside w0's storage
+        st = w0.untyped_storage()
+        adjacent = expect <= st.data_ptr() + st.nbytes()
     if adjacent:
         return w0.as_strided((n_total, k), (k, 1), w0.storage_offset())
     out = torch.empty((n_total, k), dtype=w0.dtype, device=w0.device)
@@ -379,13 +379,11 @@ class AttnProjFn(Function):
         q2 = qkv[:, : H * hd]
         k2 = qkv[:, H * hd : (H + KV) * hd]
         v2 = qkv[:, (H + KV) * hd :]
-        ld = qkv.shape[1]
         general = mask is not None or dropout_p > 0.0
         if general:
             o, lse = ops.attn_fwd_general(q2, k2, v2, B, S, H, KV, hd, scale, mask, dropout_p, seed)
         else:
-            tiles = ops.attn_path(qkv.dtype, S, hd, ld, ld, ld, H * hd) == 2
-            if not tiles and ops.attn_direct(q2, k2, v2, hd):
+            if ops.attn_direct(q2, k2, v2, hd):
                 o, lse = ops.attn_fwd_direct(q2, k2, v2, B, S, H, KV, hd, scale)
             else:
                 o, lse = ops.attn_fwd(q2, k2, v2, B, S, H, KV, hd, scale, None)
@@ -400,7 +398,6 @@ class AttnProjFn(Function):
         h2, wq, wk, wv, qkv, o, lse, cos, sin = ctx.saved_tensors
         B, S, H, KV, hd, scale = ctx.meta
         do2 = _rows(do)
-        ld = qkv.shape[1]
         dqkv = torch.empty_like(qkv)
         q2, k2, v2 = qkv[:, : H * hd], qkv[:, H * hd : (H + KV) * hd], qkv[:, (H + KV) * hd :]
         dq2, dk2, dv2 = dqkv[:, : H * hd], dqkv[:, H * hd : (H + KV) * hd], dqkv[:, (H + KV) * hd :]
@@ -409,8 +406,7 @@ class AttnProjFn(Function):
             ops.attn_bwd_general(q2, k2, v2, o, do2, lse, B, S, H, KV, hd, scale, dq2, dk2, dv2, ctx.mask,
                                  dropout_p, seed)
         else:
-            tiles = ops.attn_path(qkv.dtype, S, hd, ld, ld, ld, do2.stride(0)) == 2
-            if not tiles and ops.attn_direct(q2, k2, v2, hd, o, do2):
+            if ops.attn_direct(q2, k2, v2, hd, o, do2):
                 ops.attn_bwd_direct(q2, k2, v2, o, do2, lse, B, S, H, KV, hd, scale, dq2, dk2, dv2)
             else:
                 ops.attn_bwd(q2, k2, v2, o, do2, lse, B, S, H, KV, hd, scale, dq2, dk2, dv2)

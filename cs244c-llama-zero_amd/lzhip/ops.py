@@ -8,6 +8,7 @@ tensor or an unsupported dtype raises: there is no fallback computation.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from typing import Dict, Optional, Sequence, Tuple
 
@@ -16,6 +17,7 @@ import torch
 from . import _lib
 from ._lib import BF16, F16, F32
 
+_raw_stream = torch._C._cuda_getCurrentRawStream
 _DTYPES = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16}
 # 16-bit float formats (the MFMA GEMM and attention operands)
 HALF_DTYPES = (torch.bfloat16, torch.float16)
@@ -30,7 +32,7 @@ def dtype_code(t: torch.Tensor) -> int:
 
 def require_gpu(*tensors: Optional[torch.Tensor]) -> None:
     for t in tensors:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise RuntimeError(
                 f"llama-zero HIP kernels run on a ROCm GPU; got a tensor on {t.device}. "
                 "Move the model and inputs to 'cuda'."
@@ -38,7 +40,10 @@ def require_gpu(*tensors: Optional[torch.Tensor]) -> None:
 
 
 def stream_ptr(device: Optional[torch.device] = None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """torch's current stream on the device (default: the current one) as a
+    hipStream_t, without building a torch.cuda.Stream object for it."""
+    idx = None if device is None else device.index
+    return _raw_stream(torch.cuda.current_device() if idx is None else idx)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -49,9 +54,11 @@ def _row_stride(t: torch.Tensor) -> int:
     """Leading dimension of a 2-D row-major view (last stride must be 1)."""
     if t.dim() != 2:
         raise ValueError(f"expected a 2-D view, got shape {tuple(t.shape)}")
-    if t.stride(1) != 1 and t.size(1) > 1:
+    rows, cols = t.shape
+    ld, inner = t.stride()
+    if inner != 1 and cols > 1:
         raise ValueError("expected unit stride in the last dimension")
-    return max(t.stride(0), t.size(1)) if t.size(0) > 1 else t.size(1)
+    return max(ld, cols) if rows > 1 else cols
 
 
 # ---------------------------------------------------------------------------
@@ -456,7 +463,7 @@ def rmsnorm_bwd(x2: torch.Tensor, w: torch.Tensor, rstd: torch.Tensor, dy2: torc
     else:
         dw = torch.empty((cols,), dtype=w.dtype, device=w.device) if need_dw else None
         dw_buf = dw
-    ws = _rmsnorm_workspace(x2.device, int(_lib.load().lz_rmsnorm_bwd_workspace(rows, cols)))
+    ws = _rmsnorm_workspace(x2.device, _lib.query("lz_rmsnorm_bwd_workspace", rows, cols))
     if dres is not None:
         if dres.shape != dx.shape or dres.dtype != dx.dtype:
             raise ValueError("residual gradient must match dx")
@@ -687,17 +694,30 @@ def gemm_nt(a2: torch.Tensor, b2: torch.Tensor, out: Optional[torch.Tensor] = No
     return gemm(a2, b2, True, True, out=out, out_dtype=out_dtype, residual=residual, alpha=alpha, beta=beta)
 
 
-def _gemm_operand(t: torch.Tensor, kmajor: bool) -> Tuple[torch.Tensor, bool]:
-    """Returns (operand, kmajor) satisfying the kernel's layout rules.  A
-    K-major operand is zero-padded along K when needed (nt_operand); an
-    M/N-major operand [K, R] whose R, row stride or base is not 8-element
-    aligned is transposed into a K-major padded copy instead."""
+def _gemm_operand(t: torch.Tensor, kmajor: bool) -> Tuple[torch.Tensor, int, bool]:
+    """Returns (operand, row stride, kmajor) satisfying the kernel's layout
+    rules.  A K-major operand is zero-padded along K when needed
+    (nt_operand); an M/N-major operand [K, R] whose R, row stride or base is
+    not 8-element aligned is transposed into a K-major padded copy instead."""
     if kmajor:
-        return nt_operand(t), True
-    k, r = t.shape
-    if r % 8 == 0 and _row_stride(t) % 8 == 0 and t.data_ptr() % 16 == 0 and t.stride(-1) == 1:
-        return t, False
-    return transpose_padded(t), True
+        ld = _row_stride(t)
+        if t.shape[1] % 8 or ld % 8 or t.data_ptr() % 16:
+            t = nt_operand(t)
+            ld = _row_stride(t)
+        return t, ld, True
+    if t.stride(-1) == 1:
+        ld = _row_stride(t)
+        if t.shape[1] % 8 == 0 and ld % 8 == 0 and t.data_ptr() % 16 == 0:
+            return t, ld, False
+    t = transpose_padded(t)
+    return t, _row_stride(t), True
+
+
+@functools.lru_cache(maxsize=4096)
+def _gemm_workspace(M: int, N: int, K: int, a_kmajor: bool, b_kmajor: bool) -> int:
+    """lz_gemm_workspace, which depends on its arguments alone (the planner
+    walks a few dozen candidates: as long as the launch itself)."""
+    return int(_lib.load().lz_gemm_workspace(M, N, K, int(a_kmajor), int(b_kmajor)))
 
 
 def gemm(a: torch.Tensor, b: torch.Tensor, a_kmajor: bool = True, b_kmajor: bool = True,
@@ -710,45 +730,47 @@ def gemm(a: torch.Tensor, b: torch.Tensor, a_kmajor: bool = True, b_kmajor: bool
     dy.W is gemm(dy, W, b_kmajor=False) and dy^T.x is
     gemm(dy, x, a_kmajor=False, b_kmajor=False)."""
     require_gpu(a, b, out, residual)
-    if a.dtype == torch.float32 and b.dtype == torch.float32:
+    dtype = a.dtype
+    if dtype == torch.float32 and b.dtype == torch.float32:
         return _gemm_f32(a, b, a_kmajor, b_kmajor, out, out_dtype, residual, alpha, beta)
-    if a.dtype != b.dtype or a.dtype not in HALF_DTYPES:
+    if dtype != b.dtype or dtype not in HALF_DTYPES:
         raise TypeError(
             f"the MFMA GEMM takes two bfloat16, two float16 or two float32 operands (got {a.dtype}, {b.dtype})"
         )
-    M, K = a.shape if a_kmajor else (a.shape[1], a.shape[0])
-    N, K2 = b.shape if b_kmajor else (b.shape[1], b.shape[0])
+    M, K = a.shape if a_kmajor else a.shape[::-1]
+    N, K2 = b.shape if b_kmajor else b.shape[::-1]
     if K != K2:
         raise ValueError(f"GEMM reduction mismatch {K} vs {K2}")
-    a, a_kmajor = _gemm_operand(a, a_kmajor)
-    b, b_kmajor = _gemm_operand(b, b_kmajor)
+    a, lda, a_kmajor = _gemm_operand(a, a_kmajor)
+    b, ldb, b_kmajor = _gemm_operand(b, b_kmajor)
     if K % 8 and (a_kmajor or b_kmajor):
         # a K-major operand is zero-padded to K8: bring the other one to the same K
         if not a_kmajor:
             a, a_kmajor = transpose_padded(a), True
+            lda = _row_stride(a)
         if not b_kmajor:
             b, b_kmajor = transpose_padded(b), True
+            ldb = _row_stride(b)
     Kp = _round8(K) if (a_kmajor or b_kmajor) else K
     if out is None:
-        out = torch.empty((M, N), dtype=out_dtype or a.dtype, device=a.device)
-    if residual is not None and (residual.dtype != a.dtype or tuple(residual.shape) != (M, N)):
-        raise ValueError(f"residual must be a {a.dtype} [M, N] view")
-    lib = _lib.load()
-    ws_bytes = int(lib.lz_gemm_workspace(M, N, Kp, int(a_kmajor), int(b_kmajor)))
+        out = torch.empty((M, N), dtype=out_dtype or dtype, device=a.device)
+    if residual is not None and (residual.dtype != dtype or tuple(residual.shape) != (M, N)):
+        raise ValueError(f"residual must be a {dtype} [M, N] view")
+    ws_bytes = _gemm_workspace(M, N, Kp, bool(a_kmajor), bool(b_kmajor))
     ws = torch.empty(((ws_bytes + 15) // 16) * 4, dtype=torch.float32, device=a.device) if ws_bytes else None
     probe = _gemm_probe
     if probe is not None:
-        key = (bool(a_kmajor), bool(b_kmajor), int(lib.lz_gemm_plan(M, N, Kp, int(a_kmajor), int(b_kmajor))))
+        key = (bool(a_kmajor), bool(b_kmajor), int(_lib.load().lz_gemm_plan(M, N, Kp, int(a_kmajor), int(b_kmajor))))
         if not probe.wants(key):
             probe = None
     if probe is not None:
         start = torch.cuda.Event(enable_timing=True)
         end = torch.cuda.Event(enable_timing=True)
         start.record()
-    _lib.call("lz_gemm", a.data_ptr(), _row_stride(a), int(a_kmajor), b.data_ptr(), _row_stride(b), int(b_kmajor),
-              dtype_code(a), out.data_ptr(), _row_stride(out), dtype_code(out), _ptr(residual),
+    _lib.call("lz_gemm", a.data_ptr(), lda, int(a_kmajor), b.data_ptr(), ldb, int(b_kmajor),
+              _DTYPES[dtype], out.data_ptr(), _row_stride(out), dtype_code(out), _ptr(residual),
               _row_stride(residual) if residual is not None else 0, M, N, Kp, float(alpha), float(beta), _ptr(ws),
-              ws_bytes if ws is not None else 0, stream_ptr(a.device))
+              ws_bytes, stream_ptr(a.device))
     if probe is not None:
         end.record()
         probe.add(2.0 * M * N * K, start, end, key)
@@ -781,8 +803,7 @@ def _gemm_f32(a, b, a_kmajor, b_kmajor, out, out_dtype, residual, alpha, beta) -
         if residual.dtype != torch.float32 or tuple(residual.shape) != (M, N):
             raise ValueError("residual of a float32 GEMM must be a float32 [M, N] view")
         ldr = _unit_stride_2d(residual, "residual")
-    lib = _lib.load()
-    ws_bytes = int(lib.lz_gemm_f32_workspace(M, N, K))
+    ws_bytes = _lib.query("lz_gemm_f32_workspace", M, N, K)
     ws = torch.empty(((ws_bytes + 15) // 16) * 4, dtype=torch.float32, device=a.device) if ws_bytes else None
     probe = _gemm_probe
     if probe is not None and not probe.wants((bool(a_kmajor), bool(b_kmajor), "f32")):
@@ -803,11 +824,13 @@ def _gemm_f32(a, b, a_kmajor, b_kmajor, out, out_dtype, residual, alpha, beta) -
 def swiglu_fusable(x2: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether gemm_swiglu takes x2 [M, K] and w [2F, K]: M % 256, F % 128 and
     K % 64 == 0, bf16, unit column stride and 16-byte aligned rows."""
-    if x2.dim() != 2 or w.dim() != 2 or x2.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+    if x2.dim() != 2 or w.dim() != 2:
         return False
     M, K = x2.shape
     n2, k2 = w.shape
     if k2 != K or n2 % 256 or M % 256 or K % 64 or M == 0:
+        return False
+    if x2.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         return False
     return all(t.stride(1) == 1 and _row_stride(t) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x2, w))
 
@@ -892,11 +915,13 @@ def rope_fusable(x2: torch.Tensor, w: torch.Tensor, nrope: int, hd: int, cos: to
     nrope columns: head dim 128 or 64, M, N and nrope multiples of 256,
     K % 64 == 0, bf16, contiguous [>= S, hd] tables and 16-byte aligned
     rows."""
-    if hd not in (128, 64) or x2.dim() != 2 or w.dim() != 2 or x2.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+    if hd not in (128, 64) or x2.dim() != 2 or w.dim() != 2:
         return False
     M, K = x2.shape
     N, k2 = w.shape
     if k2 != K or M % 256 or N % 256 or K % 64 or nrope % 256 or nrope > N or M == 0:
+        return False
+    if x2.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         return False
     if cos.dtype != torch.bfloat16 or cos.dim() != 2 or cos.size(1) != hd or not cos.is_contiguous():
         return False
@@ -998,12 +1023,13 @@ def attn_fwd(q2: torch.Tensor, k2: torch.Tensor, v2: torch.Tensor, B: int, S: in
 def attn_direct(q2: torch.Tensor, k2: torch.Tensor, v2: torch.Tensor, hd: int, *rows: torch.Tensor) -> bool:
     """Whether attn_fwd_direct (rows: none) or attn_bwd_direct (rows: o, do)
     takes these row views: head dim 32, 64 or 128, 16-byte aligned rows."""
-    if q2.dtype not in _DTYPES:
+    if hd not in (32, 64, 128) or q2.dtype not in _DTYPES:
         return False
-    strides = [_row_stride(t) for t in (q2, k2, v2)]
-    lib = _lib.load()
-    return (all(t.data_ptr() % 16 == 0 for t in (q2, k2, v2, *rows))
-            and all(lib.lz_attn_direct(_DTYPES[q2.dtype], hd, *strides, _row_stride(t)) for t in (rows or (q2,))))
+    piece = 16 // q2.element_size()
+    for t in (q2, k2, v2, *rows):
+        if t.data_ptr() % 16 or _row_stride(t) % piece:
+            return False
+    return True
 
 
 def attn_fwd_direct(q2: torch.Tensor, k2: torch.Tensor, v2: torch.Tensor, B: int, S: int, H: int, KV: int, hd: int,

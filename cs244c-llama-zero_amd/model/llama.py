@@ -135,8 +135,11 @@ class RotaryEmbedding(nn.Module):
 
     def tables(self, seq_len: int, device: torch.device, dtype: torch.dtype) -> Tuple[torch.Tensor, torch.Tensor]:
         """[S, hd] views of the cache for the fused kernels."""
-        cos, sin = self.forward(seq_len, device, dtype)
-        return cos.reshape(-1, self.dim), sin.reshape(-1, self.dim)
+        cos, sin = self.cos_cached, self.sin_cached
+        if seq_len > self.max_seq_len_cached or cos.device != device or cos.dtype != dtype:
+            self._build_cache(seq_len=seq_len, device=device, dtype=dtype)
+            cos, sin = self.cos_cached, self.sin_cached
+        return cos.view(-1, self.dim).narrow(0, 0, seq_len), sin.view(-1, self.dim).narrow(0, 0, seq_len)
 
 
 class GroupedQueryAttention(nn.Module):

@@ -179,6 +179,13 @@ def flatten_param_shard_dtype(meta: FlatParamMetadata, shard_start: int, shard_e
     return _gather(meta, [p.data for p in meta.params], model_param_dtype(meta), out, shard_start, shard_start + n)
 
 
+def grad_segments(meta: FlatParamMetadata):
+    """The segment table of the parameters' current gradients, and their dtype."""
+    grads = [p.grad for p in meta.params]
+    src_dtype = next((g.dtype for g in grads if g is not None), model_param_dtype(meta))
+    return meta.segment_table(grads), src_dtype
+
+
 def flatten_grads_fp32(meta: FlatParamMetadata) -> torch.Tensor:
     return flatten_grads_dtype(meta, torch.float32)
 
@@ -190,9 +197,10 @@ def flatten_grads_dtype(meta: FlatParamMetadata, dtype: torch.dtype, out: Option
     end = meta.total_numel if end is None else end
     if out is None:
         out = torch.empty(end - begin, dtype=dtype, device=meta.device)
-    grads = [p.grad for p in meta.params]
-    src_dtype = next((g.dtype for g in grads if g is not None), model_param_dtype(meta))
-    return _gather(meta, grads, src_dtype, out, begin, end)
+    if end > begin:
+        table, src_dtype = grad_segments(meta)
+        ops.mt_gather_host(table, src_dtype, out, begin, end)
+    return out
 
 
 def assign_flat_params(meta: FlatParamMetadata, flat_params: torch.Tensor) -> None:

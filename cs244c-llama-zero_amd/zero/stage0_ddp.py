@@ -30,7 +30,7 @@ from .common import (
     bucket_ranges,
     build_flat_param_metadata,
     bytes_to_mb,
-    flatten_grads_dtype,
+    grad_segments,
     flatten_params_dtype,
     flatten_params_fp32,
     get_rank_world_size,
@@ -119,10 +119,11 @@ class ZeROStage0DDP:
         if self._flat_grads is None:
             self._flat_grads = torch.empty(self.meta.total_numel, dtype=self.param_dtype, device=self.meta.device)
         flat = self._flat_grads
+        table, src_dtype = grad_segments(self.meta)  # one table for every bucket of the step
         comm_ms = 0.0
         for b0, b1 in bucket_ranges(0, self.meta.total_numel, self.grad_bucket_numel):
             bucket = flat[b0:b1]
-            flatten_grads_dtype(self.meta, self.param_dtype, out=bucket, begin=b0, end=b1)
+            ops.mt_gather_host(table, src_dtype, bucket, b0, b1)
             t0 = time.perf_counter()
             with self.collectives.label_scope(f"{self._stage_label}.step.allreduce.grad_bucket"):
                 self.collectives.allreduce_inplace(bucket, average=False)
