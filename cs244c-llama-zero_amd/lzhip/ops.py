@@ -665,7 +665,7 @@ def gemm_kernel_name(key) -> str:
     if code == "swiglu_bwd":
         return "gemm_swiglu_bwd_kernel"
     if code == "f32":
-        return f"gemm_f32_kernel<{'true' if ak else 'false'}, {'true' if bk else 'false'}>"
+        return "gemm_f32_kernel"
     cfg, splits = code // 64, code % 64
     tf = lambda b: "true" if b else "false"
     if cfg == 5:

@@ -61,6 +61,24 @@ def test_gemm_f32_layouts_vs_float64(ak, bk, M, N, K):
     assert _rel(out, ref) <= 1e-5
 
 
+@pytest.mark.parametrize("ak,bk", [(True, True), (True, False), (False, True), (False, False)])
+@pytest.mark.parametrize("M,N,K", [
+    (31, 33, 127), (33, 64, 129), (64, 96, 260),         # 32 x 32 tiles: K in one, two and three 128-deep stages
+    (1024, 1792, 33), (1030, 1796, 100), (641, 2049, 95),  # 64 x 64: one to four 32-deep stages, ragged edges
+    (4090, 4096, 516), (4095, 4095, 257),                # 128 x 128: ragged edges, with and without 16-byte rows
+    (24, 320, 8192), (100, 132, 16420), (2056, 260, 4097),  # split: last slice short
+])
+def test_gemm_f32_tiles_and_tails_vs_float64(ak, bk, M, N, K):
+    """Each tile of the fp32 product at its edges.  A sum's error grows with
+    the 64 terms of one flush and the K/64 flushes after it: 2^-24 times
+    8 + sqrt(K / 64) bounds the rms of both walks."""
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a, b = torch.randn(M, K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    out = ops.gemm(_operand(a, ak), _operand(b, bk), ak, bk)
+    ref = a.double() @ b.double().t()
+    assert _rel(out, ref) <= 2.0 ** -24 * (8 + (K / 64) ** 0.5)
+
+
 def test_gemm_f32_split_plan():
     """Few output tiles with a long K (a language-model head's input
     gradient: 512 tokens x 256 features over a 32000 vocabulary) are split
