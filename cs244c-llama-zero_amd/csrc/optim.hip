@@ -195,6 +195,46 @@ __global__ void __launch_bounds__(kThreads) sumsq_kernel(const T* __restrict__ x
   }
 }
 
+// The 16-bit formats from 16-byte aligned rows: 16 bytes per thread and load,
+// two loads in flight, four fp32 sums per thread (the scalar kernel's 2-byte
+// loads streamed 2.2 TB/s: 100 us for the 110 M gradients of the 125M model,
+// whose ZeRO-1 step went from 731 to 684 us).
+template <typename F>
+__global__ void __launch_bounds__(kThreads) sumsq_vec16_kernel(const uint16_t* __restrict__ x, int64_t n,
+                                                               double* __restrict__ acc) {
+  __shared__ double red[kThreads / 64];
+  const uint4* xv = reinterpret_cast<const uint4*>(x);
+  const int64_t n8 = n >> 3, stride = (int64_t)gridDim.x * kThreads;
+  float part[4] = {0.f, 0.f, 0.f, 0.f};
+  auto add = [&](const uint4& q) {
+    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float a = F::to_f(w[k] & 0xffff), b = F::to_f(w[k] >> 16);
+      part[k] = fmaf(b, b, fmaf(a, a, part[k]));
+    }
+  };
+  int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  for (; i + stride < n8; i += 2 * stride) {
+    const uint4 p = xv[i], q = xv[i + stride];
+    add(p);
+    add(q);
+  }
+  if (i < n8) add(xv[i]);
+  if (blockIdx.x == 0 && (int64_t)threadIdx.x < n - 8 * n8) {
+    const float t = F::to_f(x[8 * n8 + threadIdx.x]);
+    part[0] = fmaf(t, t, part[0]);
+  }
+  const double d = wave_sum_d(((double)part[0] + (double)part[1]) + ((double)part[2] + (double)part[3]));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = d;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+    for (int w = 0; w < kThreads / 64; ++w) s += red[w];
+    atomicAdd(acc, s);
+  }
+}
+
 // Sum of the workgroup partials of adamw_vec_kernel (and the squares of the
 // n % 4 tail it leaves to the scalar kernel) added to *acc, in a fixed order:
 // kNormBlocks workgroups reduce contiguous ranges into part2, then one
@@ -896,9 +936,11 @@ LZ_EXPORT int lz_sumsq(const void* x, int dtype, int64_t n, double* acc, void* s
     if (lz_aligned16(x)) sumsq_vec4_f32_kernel<<<stream_grid(n / 4 + 1), kThreads, 0, s>>>((const float*)x, n, acc);
     else sumsq_kernel<float><<<stream_grid(n), kThreads, 0, s>>>((const float*)x, n, acc);
   } else if (dtype == LZ_BF16) {
-    sumsq_kernel<uint16_t><<<stream_grid(n), kThreads, 0, s>>>((const uint16_t*)x, n, acc);
+    if (lz_aligned16(x)) sumsq_vec16_kernel<FmtBF16><<<stream_grid(n / 8 + 1), kThreads, 0, s>>>((const uint16_t*)x, n, acc);
+    else sumsq_kernel<uint16_t><<<stream_grid(n), kThreads, 0, s>>>((const uint16_t*)x, n, acc);
   } else if (dtype == LZ_F16) {
-    sumsq_kernel<_Float16><<<stream_grid(n), kThreads, 0, s>>>((const _Float16*)x, n, acc);
+    if (lz_aligned16(x)) sumsq_vec16_kernel<FmtF16><<<stream_grid(n / 8 + 1), kThreads, 0, s>>>((const uint16_t*)x, n, acc);
+    else sumsq_kernel<_Float16><<<stream_grid(n), kThreads, 0, s>>>((const _Float16*)x, n, acc);
   } else {
     return lz_set_error(LZ_EINVAL, "lz_sumsq: bad dtype %d", dtype);
   }

@@ -1078,6 +1078,21 @@ def test_adamw_norm_matches_adamw_and_sumsq(n, gdtype, off):
         ops.adamw_norm_(pb, mb, vb, gd, acc, ws[:1], step=4, **hp)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,off", [(1, 0), (7, 0), (8, 0), (2047, 0), (4096, 0), (4104, 0), (8 * 256 * 2048 + 5, 0),
+                                   (3 * 8 * 256 * 2048 + 11, 0), (4099, 1), (4099, 8)])
+def test_sumsq_16bit_vector_edges(dtype, n, off):
+    """16-byte loads with short ends, one or several per thread, and views
+    that are not 16-byte aligned.  Each fp32 sum of a thread holds under 64
+    squares, so the total is within 64 * 2^-24 of float64."""
+    g = torch.Generator(device=DEV).manual_seed(n + off)
+    x = torch.randn(n + off, generator=g, device=DEV).to(dtype)[off:]
+    acc = torch.full((1,), 3.0, dtype=torch.float64, device=DEV)
+    ops.sumsq_(x, acc)
+    ref = float(x.double().pow(2).sum())
+    assert abs(float(acc.item()) - 3.0 - ref) <= 64 * 2.0 ** -24 * ref
+
+
 def test_sumsq_and_clip():
     g = _seed(4)
     a = torch.randn(3_000_001, generator=g)
