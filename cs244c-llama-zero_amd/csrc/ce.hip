@@ -126,11 +126,30 @@ __global__ void __launch_bounds__(1024) ce_reduce_kernel(const float* __restrict
   __shared__ double red_s[16];
   __shared__ double red_c[16];
   double acc = 0.0, cnt = 0.0;
-  for (int64_t r = threadIdx.x; r < rows; r += blockDim.x) {
-    if (row_target(labels, r, seq, vocab, ignore_index) >= 0) {
-      acc += (double)row_loss[r];
-      cnt += 1.0;
+  // Bound by the latency of one workgroup's chain of loads: four rows per
+  // thread at a time, their loads issued together and not behind a branch on
+  // the row (whose label is read one ahead, as row_target does).  The 125M head
+  // with its two passes over 16384 rows: 2845 -> 2823 us.
+  constexpr int kU = 4;
+  for (int64_t r0 = threadIdx.x; r0 < rows; r0 += kU * (int64_t)blockDim.x) {
+    int64_t t[kU];
+    float l[kU];
+    bool scored[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int64_t r = r0 + u * (int64_t)blockDim.x, i = min(r, rows - 1);
+      const bool last = seq > 0 && (rows <= 0x7fffffff && seq <= 0x7fffffff ? (uint32_t)i % (uint32_t)seq == (uint32_t)(seq - 1)
+                                                                           : i % seq == seq - 1);
+      t[u] = labels[seq > 0 && !last ? i + 1 : i];
+      l[u] = row_loss[i];
+      scored[u] = r < rows && !last;
     }
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      if (scored[u] && t[u] != ignore_index && t[u] >= 0 && t[u] < vocab) {
+        acc += (double)l[u];
+        cnt += 1.0;
+      }
   }
   acc = wave_sum_d(acc);
   cnt = wave_sum_d(cnt);
