@@ -40,8 +40,9 @@ bool lz_attn_wave_ok(const LzWaveArgs& a, int dtype, int64_t hd, bool backward);
 
 // How a call is computed.  General: mask_kind and dropout are read (also when
 // both are off, so that a call with dropout has the lse of one without);
-// otherwise causal.  bf16 probabilities and dS enter their products as two
-// bf16 terms, except with kWaveRounded (one rounding, as in the tile kernels).
+// otherwise causal.  bf16 probabilities and dS enter their products with all
+// their fp32 bits (three bf16 terms), except with kWaveRounded (one rounding,
+// as in the tile kernels).
 enum LzWaveMode { kWaveGeneral, kWaveSplit, kWaveRounded };
 
 enum LzWavePass { kWaveFwd, kWaveDq, kWaveDkdv };

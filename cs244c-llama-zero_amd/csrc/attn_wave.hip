@@ -27,8 +27,11 @@
 //   PolF32: fp32 MFMAs (v_mfma_f32_32x32x2_f32) on fp32 tiles; fp32 and fp16
 //     operands.  Every value after the load is fp32.
 //   PolBF16: bf16 MFMAs on bf16 tiles.  The fp32 weights (probabilities, dS)
-//     enter cols() as two bf16 terms (kSplit: value = hi + lo to 2^-17, two
-//     MFMAs) or rounded to bf16 once, as the tile kernels of attn.hip do.
+//     enter cols() as three bf16 terms that add up to them exactly (kSplit: 24
+//     bits in pieces of eight, three MFMAs) or rounded to bf16 once, as the tile
+//     kernels of attn.hip do.
+// kExact policies keep fp32 values fp32 from the score to the last product:
+// natural units and exp_accurate, no rounded weights.
 #include "attn_wave.h"
 
 #include "attn_tiles.h"
@@ -59,7 +62,7 @@ __device__ __forceinline__ float exp_accurate(float d) {
 template <typename T, int HD_>
 struct PolF32 {
   static constexpr int HD = HD_;
-  static constexpr bool kF32 = true;
+  static constexpr bool kExact = true, k16 = false;  // k16: 16-bit tiles
   static constexpr int RS = HD + 4, kTile = 32 * RS * 4;
   static constexpr int kPieces = HD / 8;  // 4-element pieces of a tile per lane
   typedef T Ptr;
@@ -167,9 +170,10 @@ struct PolF32 {
 template <int HD_, bool kSplit>
 struct PolBF16 {
   static constexpr int HD = HD_;
-  static constexpr bool kF32 = false;
+  static constexpr bool kExact = kSplit, k16 = true;
   static constexpr int kTile = 32 * HD * 2;
   static constexpr int kPieces = HD / 16;  // 8-element pieces of a tile per lane
+  static constexpr int kTerms = kSplit ? 3 : 1;
   typedef uint16_t Ptr;
 
   struct Own {
@@ -228,21 +232,30 @@ struct PolBF16 {
                                               const f32x16_t& p) {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      uint32_t hw[4], lw[4];
+      uint32_t w[kTerms][4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float p0 = p[8 * ks + 2 * e], p1 = p[8 * ks + 2 * e + 1];
-        hw[e] = pack_bf16x2(p0, p1);
-        if constexpr (kSplit)
-          lw[e] = pack_bf16x2(p0 - __uint_as_float(hw[e] << 16), p1 - __uint_as_float(hw[e] & 0xffff0000u));
+        float p0 = p[8 * ks + 2 * e], p1 = p[8 * ks + 2 * e + 1];
+        if constexpr (kSplit) {
+          // the top eight significant bits of what is left, cut and not
+          // rounded: each remainder is exact and the third has at most eight
+#pragma unroll
+          for (int t = 0; t < kTerms; ++t) {
+            const uint32_t b0 = __float_as_uint(p0), b1 = __float_as_uint(p1);
+            w[t][e] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+            p0 -= __uint_as_float(b0 & 0xffff0000u);
+            p1 -= __uint_as_float(b1 & 0xffff0000u);
+          }
+        } else {
+          w[0][e] = pack_bf16x2(p0, p1);
+        }
       }
-      const bf16x8_t ph = __builtin_bit_cast(bf16x8_t, make_uint4(hw[0], hw[1], hw[2], hw[3]));
 #pragma unroll
       for (int i = 0; i < HD / 32; ++i) {
         const bf16x8_t f = cx.to.frag_t(tile, ks, i);
-        acc[i] = mfma16<FmtBF16>(f, ph, acc[i]);
-        if constexpr (kSplit)
-          acc[i] = mfma16<FmtBF16>(f, __builtin_bit_cast(bf16x8_t, make_uint4(lw[0], lw[1], lw[2], lw[3])), acc[i]);
+#pragma unroll
+        for (int t = kTerms - 1; t >= 0; --t)  // the smallest first
+          acc[i] = mfma16<FmtBF16>(f, __builtin_bit_cast(bf16x8_t, make_uint4(w[t][0], w[t][1], w[t][2], w[t][3])), acc[i]);
       }
     }
   }
@@ -251,17 +264,16 @@ struct PolBF16 {
   }
 };
 
-// Units of the running maximum and of exp: natural for fp32 and for masks
-// (score + mask must not be scaled to log2 units: a mask of the type's lowest
-// value would overflow), log2 for plain causal bf16.
-template <class P, bool kGen>
+// Units of the running maximum and of exp: natural for the exact policies (a
+// mask of the type's lowest value would overflow in log2 units too), log2 for
+// rounded causal bf16.
+template <class P>
 __device__ __forceinline__ float score_unit(float scale) {
-  return (P::kF32 || kGen) ? scale : scale * kLog2e;
+  return P::kExact ? scale : scale * kLog2e;
 }
-template <class P, bool kGen>
+template <class P>
 __device__ __forceinline__ float exp_unit(float d) {
-  if constexpr (P::kF32) return exp_accurate(d);
-  else if constexpr (kGen) return __builtin_amdgcn_exp2f(d * kLog2e);
+  if constexpr (P::kExact) return exp_accurate(d);
   else return __builtin_amdgcn_exp2f(d);
 }
 
@@ -396,7 +408,7 @@ __global__ void __launch_bounds__(64 * NW) attn_fwd_wave_kernel(LzWaveArgs a) {
   const void* vbase = row_ptr<P>(a.v, (int64_t)b * S, a.ldv, (int64_t)g * HD);
   const bool masked = kGen && a.mask_kind != 0;
   const int nt = masked ? nqt : qb + 1;
-  const float u = score_unit<P, kGen>(a.scale);
+  const float u = score_unit<P>(a.scale);
   const int64_t moff = (int64_t)b * a.msb + (int64_t)h * a.msh + (int64_t)qc * a.msq;
 
   f32x16_t o[HD / 32];
@@ -461,12 +473,12 @@ __global__ void __launch_bounds__(64 * NW) attn_fwd_wave_kernel(LzWaveArgs a) {
     mx = max_halves(mx);
     const float m_new = fmaxf(m, mx);
     const float ms = m_new == -INFINITY ? 0.f : m_new;  // nothing seen yet: every term below is exp(-inf)
-    const float alpha = exp_unit<P, kGen>(m - ms);
+    const float alpha = exp_unit<P>(m - ms);
     m = m_new;
     float rs = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = exp_unit<P, kGen>(s[r] - ms);
+      s[r] = exp_unit<P>(s[r] - ms);
       rs += s[r];
     }
     l = l * alpha + sum_halves(rs);
@@ -497,7 +509,7 @@ __global__ void __launch_bounds__(64 * NW) attn_fwd_wave_kernel(LzWaveArgs a) {
   float f[NW], L = 0.f;
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
-    f[w] = exp_unit<P, kGen>(ml[w][l32] - Ms);
+    f[w] = exp_unit<P>(ml[w][l32] - Ms);
     L = fmaf(f[w], ml[w][l32 + 32], L);
   }
   const float inv = 1.f / L;  // a row with every key masked: 0 * inf = NaN
@@ -515,7 +527,7 @@ __global__ void __launch_bounds__(64 * NW) attn_fwd_wave_kernel(LzWaveArgs a) {
   }
   if (wave == 0 && half == 0 && qrow < S) {
     float lse;
-    if constexpr (P::kF32 || kGen) lse = M + logf(L);
+    if constexpr (P::kExact) lse = M + logf(L);
     else lse = (M + log2f(L)) * kLn2;
     a.lse[((int64_t)b * H + h) * S + qrow] = lse;
   }
@@ -552,12 +564,12 @@ __global__ void __launch_bounds__(64 * NW) attn_dq_wave_kernel(LzWaveArgs a) {
     D = a.delta[li];
   }
   const float lse = a.lse[li];
-  const float lu = (P::kF32 || kGen) ? lse : lse * kLog2e;
+  const float lu = P::kExact ? lse : lse * kLog2e;
   const void* kbase = row_ptr<P>(a.k, (int64_t)b * S, a.ldk, (int64_t)g * HD);
   const void* vbase = row_ptr<P>(a.v, (int64_t)b * S, a.ldv, (int64_t)g * HD);
   const bool masked = kGen && a.mask_kind != 0;
   const int nt = masked ? nqt : qb + 1;
-  const float u = score_unit<P, kGen>(a.scale);
+  const float u = score_unit<P>(a.scale);
   const int64_t moff = (int64_t)b * a.msb + (int64_t)h * a.msh + (int64_t)qc * a.msq;
   // a query whose keys are all masked (lse -inf) has NaN gradients: its tiles are never skipped
   const bool may_skip = __ballot(lse == -INFINITY) == 0;
@@ -598,7 +610,7 @@ __global__ void __launch_bounds__(64 * NW) attn_dq_wave_kernel(LzWaveArgs a) {
       const int kv = kv0 + 8 * (r >> 2) + 4 * half + (r & 3);
       float x = s[r] * u;
       if (masked) x = mb[r] == -INFINITY ? -INFINITY : x + mb[r];
-      const float p = exp_unit<P, kGen>(x - lu);
+      const float p = exp_unit<P>(x - lu);
       float z = 1.f;
       if constexpr (kGen) {
         if (a.drop_thresh) z = drop_of(a, b, h, qc, kv);
@@ -643,7 +655,7 @@ __global__ void __launch_bounds__(64 * NW) attn_dkdv_wave_kernel(LzWaveArgs a) {
   P::load_own(vf, row_ptr<P>(a.v, grow, a.ldv, (int64_t)g * HD), half);
   const bool masked = kGen && a.mask_kind != 0;
   const int first = masked ? 0 : kb, per = nqt - first, items = rep * per;
-  const float u = score_unit<P, kGen>(a.scale);
+  const float u = score_unit<P>(a.scale);
 
   f32x16_t dk[HD / 32], dv[HD / 32];
   zero_acc(dk);
@@ -692,7 +704,7 @@ __global__ void __launch_bounds__(64 * NW) attn_dkdv_wave_kernel(LzWaveArgs a) {
         const int r = 4 * r4 + e;
         float x = s[r] * u;
         if (masked) x = mb[r] == -INFINITY ? -INFINITY : x + mb[r];
-        const float p = exp_unit<P, kGen>(x - ((P::kF32 || kGen) ? lv[e] : lv[e] * kLog2e));
+        const float p = exp_unit<P>(x - (P::kExact ? lv[e] : lv[e] * kLog2e));
         float z = 1.f;
         if constexpr (kGen) {
           if (a.drop_thresh) z = drop_of(a, b, h, q0 + 8 * r4 + 4 * half + e, kvc);
@@ -732,7 +744,7 @@ __global__ void __launch_bounds__(64 * NW) attn_dkdv_wave_kernel(LzWaveArgs a) {
 // the registers of two waves per SIMD suffice, four otherwise.
 template <class P>
 constexpr int waves_of() {
-  return P::HD == 32 || (P::HD == 64 && !P::kF32) ? 8 : 4;
+  return P::HD == 32 || (P::HD == 64 && P::k16) ? 8 : 4;
 }
 
 template <class P, bool kGen>

@@ -1,0 +1,82 @@
+"""Attention calls whose weights are fp32 from the scores to the last product
+(fp32 and ragged fp16 operands, bf16 heads of 32, explicit masks, dropout)."""
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from lzhip import ops
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+def _heads(t, B, S, n, hd):
+    return t.double().cpu().view(B, S, n, hd).transpose(1, 2)
+
+
+def _call(qkv, do, B, S, H, KV, hd, mask, p=0.0, key=0):
+    """(o, lse, dq, dk, dv) through the entry points the layer takes."""
+    q2, k2, v2 = qkv[:, : H * hd], qkv[:, H * hd : (H + KV) * hd], qkv[:, (H + KV) * hd :]
+    d = torch.zeros_like(qkv)
+    grads = d[:, : H * hd], d[:, H * hd : (H + KV) * hd], d[:, (H + KV) * hd :]
+    scale = hd**-0.5
+    if mask is None and p == 0.0:
+        o, lse = ops.attn_fwd_direct(q2, k2, v2, B, S, H, KV, hd, scale)
+        ops.attn_bwd_direct(q2, k2, v2, o, do, lse, B, S, H, KV, hd, scale, *grads)
+    else:
+        o, lse = ops.attn_fwd_general(q2, k2, v2, B, S, H, KV, hd, scale, mask, p, key)
+        ops.attn_bwd_general(q2, k2, v2, o, do, lse, B, S, H, KV, hd, scale, *grads, mask, p, key)
+    return o, lse, *grads
+
+
+@pytest.mark.parametrize("masked,hd", [(False, 32), (True, 32), (True, 64), (True, 128)])
+def test_bf16_weights_keep_their_fp32_bits(masked, hd):
+    """Every output is a difference of nearly equal probabilities: keys come
+    in pairs (one bf16 ulp apart in one small column, V of opposite sign) and
+    so do queries (dO of opposite sign), so O, dQ, dK and dV are about 1e-4 of
+    the weights they are formed from.  Rounding an output to bf16 costs
+    2^-9 / sqrt(3) of it (0.11 %), weights good to a few fp32 ulps
+    4 * 2^-24 / 1e-4 (0.24 %); weights of 17 bits would cost 2 %."""
+    S, n = 64, 32  # keys below n, queries from n on: every query sees every key
+    g = torch.Generator().manual_seed(hd + masked)
+    q, k, v, do = (torch.zeros(S, hd) for _ in range(4))
+
+    def pairs(rows, small, step):
+        x = torch.randn(n // 2, hd, generator=g).to(BF16).float()
+        x[:, small] = {32: 0.0625, 64: 0.09375, 128: 0.125}[hd] * (1 - 2 * torch.randint(0, 2, (n // 2,), generator=g))
+        x[:, step] = 1.0
+        y = x.clone()
+        y[:, step] = 1.0 + 2.0**-7
+        rows.view(n // 2, 2, hd)[:] = torch.stack([x, y], 1)
+
+    def signs(rows):
+        x = torch.randn(n // 2, hd, generator=g)
+        rows.view(n // 2, 2, hd)[:] = torch.stack([x, -x], 1)
+
+    pairs(k[:n], small=0, step=1)
+    pairs(q[n:], small=1, step=0)
+    signs(v[:n])
+    signs(do[n:])
+    k[n:] = torch.randn(S - n, hd, generator=g)
+    q[:n] = torch.randn(n, hd, generator=g)
+    q, k, v, do = (t.to(BF16) for t in (q, k, v, do))
+    mask = None
+    if masked:  # the same pairs, as a mask
+        mask = ~torch.triu(torch.ones(S, S, dtype=torch.bool, device=DEV), 1)
+    o, lse, dq, dk, dv = _call(torch.cat([q, k, v], 1).to(DEV), do.to(DEV), 1, S, 1, 1, hd, mask)
+
+    scale = hd**-0.5
+    Q, K, V, dO, O = (t.double().cpu() for t in (q, k, v, do, o))
+    s = (Q @ K.t()) * scale
+    s = s.masked_fill(torch.triu(torch.ones(S, S, dtype=torch.bool), 1), -math.inf)
+    P = torch.softmax(s, -1)
+    assert float((lse.cpu()[0, 0].double() - torch.logsumexp(s, -1)).abs().max()) < 1e-6
+    dS = P * (dO @ V.t() - (dO * O).sum(-1, keepdim=True))  # delta from the rounded O, as the kernels form it
+    want = {"o": (P @ V)[n:], "dq": scale * (dS @ K)[n:], "dk": scale * (dS.t() @ Q)[:n], "dv": (P.t() @ dO)[:n]}
+    got = {"o": o[n:], "dq": dq[n:], "dk": dk[:n], "dv": dv[:n]}
+    err = {key: float((got[key].cpu().double() - w).norm() / w.norm()) for key, w in want.items()}
+    assert max(err.values()) < 0.005, err
