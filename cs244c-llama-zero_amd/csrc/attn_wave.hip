@@ -31,8 +31,14 @@
 //     bits in pieces of eight, three MFMAs) or rounded to bf16 once, as the tile
 //     kernels of attn.hip do.
 // kExact policies keep fp32 values fp32 from the score to the last product:
-// natural units and exp_accurate, no rounded weights.
+// natural units and exp_accurate, no rounded weights.  In their products a row
+// that an owned one does not see has weight 0, and 0 * inf is NaN (as is a
+// zero term of a split weight times a visible inf), so a wave whose sums are
+// not finite goes over its tiles again with cols_seen(), which leaves unseen
+// rows out; finite inputs never do.
 #include "attn_wave.h"
+
+#include <type_traits>
 
 #include "attn_tiles.h"
 
@@ -130,8 +136,8 @@ struct PolF32 {
       *reinterpret_cast<float4*>(tile + (r * RS + col) * 4) = v;
     }
   }
-  static __device__ __forceinline__ void zero_row(char* tile, int r, int lane) {
-    if (lane < HD / 4) *reinterpret_cast<float4*>(tile + (r * RS + 4 * lane) * 4) = make_float4(0.f, 0.f, 0.f, 0.f);
+  static __device__ __forceinline__ float elem(const char* tile, int r, int c) {
+    return *reinterpret_cast<const float*>(tile + (r * RS + c) * 4);
   }
   struct Ctx {
     int row, col;  // byte offsets of this lane's rows() and cols() reads
@@ -217,8 +223,8 @@ struct PolBF16 {
       *reinterpret_cast<uint4*>(tile + toff<HD>(r, p % (HD / 8))) = row0 + r < S ? st.p[i] : make_uint4(0, 0, 0, 0);
     }
   }
-  static __device__ __forceinline__ void zero_row(char* tile, int r, int lane) {
-    if (lane < HD / 8) *reinterpret_cast<uint4*>(tile + toff<HD>(r, lane)) = make_uint4(0, 0, 0, 0);
+  static __device__ __forceinline__ float elem(const char* tile, int r, int c) {
+    return bf2f(*reinterpret_cast<const uint16_t*>(tile + toff<HD>(r, c >> 3) + (c & 7) * 2));
   }
   struct Ctx {
     TileOffsets<HD> to;
@@ -356,6 +362,50 @@ __device__ __forceinline__ void zero_acc(f32x16_t (&acc)[N]) {
     for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
 }
 
+// A tile straight into LDS (the second pass stages nothing ahead, so that it
+// does not raise the kernel's registers).
+template <class P>
+__device__ __forceinline__ void copy_tile(const void* base, int64_t ld, char* tile, int row0, int S, int lane) {
+  typename P::Stage st;
+  P::load(st, base, ld, row0, S, lane);
+  P::store(st, tile, row0, S, lane);
+}
+
+template <int N>
+__device__ __forceinline__ bool all_finite(const f32x16_t (&acc)[N]) {
+  float z = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) z = fmaf(acc[i][r], 0.f, z);
+  return __ballot(!(z == 0.f)) == 0;
+}
+
+// P::cols() one row of the tile at a time with fp32 multiply-adds, without the
+// rows r of `hidden` (bit r: this lane's owned row does not see register r's).
+template <class P>
+__device__ __forceinline__ void cols_seen(f32x16_t (&acc)[P::HD / 32], const char* tile, const f32x16_t& w,
+                                          uint32_t hidden, int lane) {
+  const int l32 = lane & 31, half = lane >> 5;
+#pragma unroll 1
+  for (int row = 0; row < 32; ++row) {
+    const int r = 4 * (row >> 3) + (row & 3), from = l32 + 8 * (row & 4);  // the lane whose register r is this row
+    float x = w[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) x = e == r ? w[e] : x;
+    x = __shfl(x, from, 64);
+    const bool skip = (__shfl((int)hidden, from, 64) >> r) & 1;
+#pragma unroll
+    for (int i = 0; i < P::HD / 32; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float y = fmaf(x, P::elem(tile, row, 32 * i + 8 * (e >> 2) + 4 * half + (e & 3)), acc[i][e]);
+        acc[i][e] = skip ? acc[i][e] : y;
+        if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // few reads in flight: few registers
+      }
+  }
+}
+
 // This wave's accumulators into its LDS region as [register][lane].
 template <int N>
 __device__ __forceinline__ void park_acc(char* region, const f32x16_t (&acc)[N], int lane) {
@@ -412,88 +462,92 @@ __global__ void __launch_bounds__(64 * NW) attn_fwd_wave_kernel(LzWaveArgs a) {
   const int64_t moff = (int64_t)b * a.msb + (int64_t)h * a.msh + (int64_t)qc * a.msq;
 
   f32x16_t o[HD / 32];
-  zero_acc(o);
-  float m = -INFINITY, l = 0.f;
-  typename P::Stage ks, vs;
-  if (wave < nt) {
-    P::load(ks, kbase, a.ldk, wave * 32, S, lane);
-    P::load(vs, vbase, a.ldv, wave * 32, S, lane);
-  }
-  for (int t = wave; t < nt; t += NW) {
-    const int kv0 = t * 32;
-    P::store(ks, Kt, kv0, S, lane);
-    P::store(vs, Vt, kv0, S, lane);
-    wave_order();
-    if (t + NW < nt) {
-      P::load(ks, kbase, a.ldk, kv0 + 32 * NW, S, lane);
-      P::load(vs, vbase, a.ldv, kv0 + 32 * NW, S, lane);
+  float m, l;
+  auto pass = [&](auto seen_only) {
+    zero_acc(o);
+    m = -INFINITY;
+    l = 0.f;
+    typename P::Stage ks, vs;
+    if (!seen_only && wave < nt) {
+      P::load(ks, kbase, a.ldk, wave * 32, S, lane);
+      P::load(vs, vbase, a.ldv, wave * 32, S, lane);
     }
-    float mb[16];
-    bool bool_holes = false;
-    if constexpr (kGen) {
+    for (int t = wave; t < nt; t += NW) {
+      const int kv0 = t * 32;
+      if constexpr (seen_only) {
+        copy_tile<P>(kbase, a.ldk, Kt, kv0, S, lane);
+        copy_tile<P>(vbase, a.ldv, Vt, kv0, S, lane);
+      } else {
+        P::store(ks, Kt, kv0, S, lane);
+        P::store(vs, Vt, kv0, S, lane);
+      }
+      wave_order();
+      if (!seen_only && t + NW < nt) {
+        P::load(ks, kbase, a.ldk, kv0 + 32 * NW, S, lane);
+        P::load(vs, vbase, a.ldv, kv0 + 32 * NW, S, lane);
+      }
+      float mb[16];
+      if constexpr (kGen) {
+        if (masked) {
+          mask_of_query(a, mb, moff, kv0, half);
+          if (a.mask_kind == 1 && all_lanes_masked(mb)) continue;  // no query of this wave sees these keys
+        }
+      }
+      f32x16_t s;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = 0.f;
+      P::rows(cx, s, Kt, qf);
       if (masked) {
-        mask_of_query(a, mb, moff, kv0, half);
-        if (a.mask_kind == 1) {
-          if (all_lanes_masked(mb)) continue;  // no query of this wave sees these keys
-          bool_holes = true;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = mb[r] == -INFINITY ? -INFINITY : fmaf(s[r], u, mb[r]);
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] *= u;
+        if (t == qb) {  // the diagonal tile (and the last one: keys past S lie past every query)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (kv0 + 8 * (r >> 2) + 4 * half + (r & 3) > qrow) s[r] = -INFINITY;
         }
       }
-    }
-    f32x16_t s;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = 0.f;
-    P::rows(cx, s, Kt, qf);
-    if (masked) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = mb[r] == -INFINITY ? -INFINITY : fmaf(s[r], u, mb[r]);
-      if (bool_holes) {
-        // rows of V that every query of this wave hides (padding) must not
-        // reach the product as 0 * inf
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const uint64_t seen = __ballot(mb[r] > -INFINITY);
-          const int row = 8 * (r >> 2) + (r & 3);
-          if ((uint32_t)seen == 0) P::zero_row(Vt, row, lane);
-          if ((uint32_t)(seen >> 32) == 0) P::zero_row(Vt, row + 4, lane);
-        }
-        wave_order();
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] *= u;
-      if (t == qb) {  // the diagonal tile (and the last one: keys past S lie past every query)
+      uint32_t hidden = 0;
+      if constexpr (seen_only) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          if (kv0 + 8 * (r >> 2) + 4 * half + (r & 3) > qrow) s[r] = -INFINITY;
+          hidden |= (masked ? s[r] == -INFINITY : kv0 + 8 * (r >> 2) + 4 * half + (r & 3) > qrow) ? 1u << r : 0u;
       }
-    }
-    float mx = s[0];
+      float mx = s[0];
 #pragma unroll
-    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
-    mx = max_halves(mx);
-    const float m_new = fmaxf(m, mx);
-    const float ms = m_new == -INFINITY ? 0.f : m_new;  // nothing seen yet: every term below is exp(-inf)
-    const float alpha = exp_unit<P>(m - ms);
-    m = m_new;
-    float rs = 0.f;
+      for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+      mx = max_halves(mx);
+      const float m_new = fmaxf(m, mx);
+      const float ms = m_new == -INFINITY ? 0.f : m_new;  // nothing seen yet: every term below is exp(-inf)
+      const float alpha = exp_unit<P>(m - ms);
+      m = m_new;
+      float rs = 0.f;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s[r] = exp_unit<P>(s[r] - ms);
-      rs += s[r];
-    }
-    l = l * alpha + sum_halves(rs);
-    if constexpr (kGen) {
-      if (a.drop_thresh) {  // the normaliser sums the probabilities before dropout
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] *= drop_of(a, b, h, qc, kv0 + 8 * (r >> 2) + 4 * half + (r & 3));
+      for (int r = 0; r < 16; ++r) {
+        s[r] = exp_unit<P>(s[r] - ms);
+        rs += s[r];
       }
+      l = l * alpha + sum_halves(rs);
+      if constexpr (kGen) {
+        if (a.drop_thresh) {  // the normaliser sums the probabilities before dropout
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[r] *= drop_of(a, b, h, qc, kv0 + 8 * (r >> 2) + 4 * half + (r & 3));
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < HD / 32; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
+      if constexpr (seen_only) cols_seen<P>(o, Vt, s, hidden, lane);
+      else P::cols(cx, o, Vt, s);
+      wave_order();  // the next tile's stores stay behind these reads
     }
-#pragma unroll
-    for (int i = 0; i < HD / 32; ++i)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
-    P::cols(cx, o, Vt, s);
-    wave_order();  // the next tile's stores stay behind these reads
+  };
+  pass(std::false_type{});
+  if constexpr (P::kExact) {
+    if (!all_finite(o)) pass(std::true_type{});
   }
   wave_order();
   park_acc(Kt, o, lane);
@@ -575,56 +629,77 @@ __global__ void __launch_bounds__(64 * NW) attn_dq_wave_kernel(LzWaveArgs a) {
   const bool may_skip = __ballot(lse == -INFINITY) == 0;
 
   f32x16_t dq[HD / 32];
-  zero_acc(dq);
-  typename P::Stage ks, vs;
-  if (wave < nt) {
-    P::load(ks, kbase, a.ldk, wave * 32, S, lane);
-    P::load(vs, vbase, a.ldv, wave * 32, S, lane);
-  }
-  for (int t = wave; t < nt; t += NW) {
-    const int kv0 = t * 32;
-    P::store(ks, Kt, kv0, S, lane);
-    P::store(vs, Vt, kv0, S, lane);
-    wave_order();
-    if (t + NW < nt) {
-      P::load(ks, kbase, a.ldk, kv0 + 32 * NW, S, lane);
-      P::load(vs, vbase, a.ldv, kv0 + 32 * NW, S, lane);
+  auto pass = [&](auto seen_only) {
+    zero_acc(dq);
+    typename P::Stage ks, vs;
+    if (!seen_only && wave < nt) {
+      P::load(ks, kbase, a.ldk, wave * 32, S, lane);
+      P::load(vs, vbase, a.ldv, wave * 32, S, lane);
     }
-    float mb[16];
-    if constexpr (kGen) {
-      if (masked) {
-        mask_of_query(a, mb, moff, kv0, half);
-        if (a.mask_kind == 1 && may_skip && all_lanes_masked(mb)) continue;
+    for (int t = wave; t < nt; t += NW) {
+      const int kv0 = t * 32;
+      if constexpr (seen_only) {
+        copy_tile<P>(kbase, a.ldk, Kt, kv0, S, lane);
+        copy_tile<P>(vbase, a.ldv, Vt, kv0, S, lane);
+      } else {
+        P::store(ks, Kt, kv0, S, lane);
+        P::store(vs, Vt, kv0, S, lane);
       }
-    }
-    f32x16_t s, dp;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s[r] = 0.f;
-      dp[r] = 0.f;
-    }
-    P::rows(cx, s, Kt, qf);
-    P::rows(cx, dp, Vt, df);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int kv = kv0 + 8 * (r >> 2) + 4 * half + (r & 3);
-      float x = s[r] * u;
-      if (masked) x = mb[r] == -INFINITY ? -INFINITY : x + mb[r];
-      const float p = exp_unit<P>(x - lu);
-      float z = 1.f;
+      wave_order();
+      if (!seen_only && t + NW < nt) {
+        P::load(ks, kbase, a.ldk, kv0 + 32 * NW, S, lane);
+        P::load(vs, vbase, a.ldv, kv0 + 32 * NW, S, lane);
+      }
+      float mb[16];
       if constexpr (kGen) {
-        if (a.drop_thresh) z = drop_of(a, b, h, qc, kv);
+        if (masked) {
+          mask_of_query(a, mb, moff, kv0, half);
+          if (a.mask_kind == 1 && may_skip && all_lanes_masked(mb)) continue;
+        }
       }
-      dp[r] = p * (fmaf(z, dp[r], -D));
-    }
-    if (masked ? kv0 + 32 > S : t == qb) {
-      const int last = masked ? S - 1 : qrow;
+      f32x16_t s, dp;
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (kv0 + 8 * (r >> 2) + 4 * half + (r & 3) > last) dp[r] = 0.f;
+      for (int r = 0; r < 16; ++r) {
+        s[r] = 0.f;
+        dp[r] = 0.f;
+      }
+      P::rows(cx, s, Kt, qf);
+      P::rows(cx, dp, Vt, df);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int kv = kv0 + 8 * (r >> 2) + 4 * half + (r & 3);
+        float x = s[r] * u;
+        if (masked) x = mb[r] == -INFINITY ? -INFINITY : x + mb[r];
+        const float p = exp_unit<P>(x - lu);
+        float z = 1.f;
+        if constexpr (kGen) {
+          if (a.drop_thresh) z = drop_of(a, b, h, qc, kv);
+        }
+        dp[r] = p * (fmaf(z, dp[r], -D));
+      }
+      if (masked ? kv0 + 32 > S : t == qb) {
+        const int last = masked ? S - 1 : qrow;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (kv0 + 8 * (r >> 2) + 4 * half + (r & 3) > last) dp[r] = 0.f;
+      }
+      if constexpr (seen_only) {
+        uint32_t hidden = 0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int kv = kv0 + 8 * (r >> 2) + 4 * half + (r & 3);
+          hidden |= (masked ? kv >= S || (mb[r] == -INFINITY && lse != -INFINITY) : kv > qrow) ? 1u << r : 0u;
+        }
+        cols_seen<P>(dq, Kt, dp, hidden, lane);
+      } else {
+        P::cols(cx, dq, Kt, dp);
+      }
+      wave_order();
     }
-    P::cols(cx, dq, Kt, dp);
-    wave_order();
+  };
+  pass(std::false_type{});
+  if constexpr (P::kExact) {
+    if (!all_finite(dq)) pass(std::true_type{});
   }
   wave_order();
   park_acc(Kt, dq, lane);
@@ -658,76 +733,101 @@ __global__ void __launch_bounds__(64 * NW) attn_dkdv_wave_kernel(LzWaveArgs a) {
   const float u = score_unit<P>(a.scale);
 
   f32x16_t dk[HD / 32], dv[HD / 32];
-  zero_acc(dk);
-  zero_acc(dv);
-  typename P::Stage qs, ds;
-  float row_val = 0.f;
-  auto fetch = [&](int it) {
-    const int hq = it / per, q0 = (first + it - hq * per) * 32, h = g * rep + hq;
-    P::load(qs, row_ptr<P>(a.q, (int64_t)b * S, a.ldq, (int64_t)h * HD), a.ldq, q0, S, lane);
-    P::load(ds, row_ptr<P>(a.dout, (int64_t)b * S, a.lddo, (int64_t)h * HD), a.lddo, q0, S, lane);
-    const int64_t li = ((int64_t)b * H + h) * S + min(q0 + l32, S - 1);
-    row_val = half == 0 ? a.lse[li] : a.delta[li];
-  };
-  if (wave < items) fetch(wave);
-  for (int it = wave; it < items; it += NW) {
-    const int hq = it / per, qt = first + it - hq * per, q0 = qt * 32, h = g * rep + hq;
-    P::store(qs, Qt, q0, S, lane);
-    P::store(ds, Dt, q0, S, lane);
-    rows_s[wave][lane] = row_val;
-    const bool finite_rows = __ballot(half == 0 && row_val == -INFINITY) == 0;
-    wave_order();
-    if (it + NW < items) fetch(it + NW);
-    float mb[16];
-    if constexpr (kGen) {
-      if (masked) {
-        mask_of_key(a, mb, (int64_t)b * a.msb + (int64_t)h * a.msh + (int64_t)kvc * a.msk, q0, half);
-        if (a.mask_kind == 1 && finite_rows && all_lanes_masked(mb)) continue;
+  auto pass = [&](auto seen_only) {
+    zero_acc(dk);
+    zero_acc(dv);
+    typename P::Stage qs, ds;
+    float row_val = 0.f;
+    auto row_value = [&](int h, int q0) {
+      const int64_t li = ((int64_t)b * H + h) * S + min(q0 + l32, S - 1);
+      return half == 0 ? a.lse[li] : a.delta[li];
+    };
+    auto fetch = [&](int it) {
+      const int hq = it / per, q0 = (first + it - hq * per) * 32, h = g * rep + hq;
+      P::load(qs, row_ptr<P>(a.q, (int64_t)b * S, a.ldq, (int64_t)h * HD), a.ldq, q0, S, lane);
+      P::load(ds, row_ptr<P>(a.dout, (int64_t)b * S, a.lddo, (int64_t)h * HD), a.lddo, q0, S, lane);
+      row_val = row_value(h, q0);
+    };
+    if (!seen_only && wave < items) fetch(wave);
+    for (int it = wave; it < items; it += NW) {
+      const int hq = it / per, qt = first + it - hq * per, q0 = qt * 32, h = g * rep + hq;
+      if constexpr (seen_only) {
+        copy_tile<P>(row_ptr<P>(a.q, (int64_t)b * S, a.ldq, (int64_t)h * HD), a.ldq, Qt, q0, S, lane);
+        copy_tile<P>(row_ptr<P>(a.dout, (int64_t)b * S, a.lddo, (int64_t)h * HD), a.lddo, Dt, q0, S, lane);
+        row_val = row_value(h, q0);
+      } else {
+        P::store(qs, Qt, q0, S, lane);
+        P::store(ds, Dt, q0, S, lane);
       }
-    }
-    f32x16_t s, dp;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s[r] = 0.f;
-      dp[r] = 0.f;
-    }
-    P::rows(cx, s, Qt, kf);
-    P::rows(cx, dp, Dt, vf);
-    f32x16_t pz;
-#pragma unroll
-    for (int r4 = 0; r4 < 4; ++r4) {
-      const float4 l4 = *reinterpret_cast<const float4*>(&rows_s[wave][8 * r4 + 4 * half]);
-      const float4 d4 = *reinterpret_cast<const float4*>(&rows_s[wave][32 + 8 * r4 + 4 * half]);
-      const float lv[4] = {l4.x, l4.y, l4.z, l4.w}, dl[4] = {d4.x, d4.y, d4.z, d4.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int r = 4 * r4 + e;
-        float x = s[r] * u;
-        if (masked) x = mb[r] == -INFINITY ? -INFINITY : x + mb[r];
-        const float p = exp_unit<P>(x - (P::kExact ? lv[e] : lv[e] * kLog2e));
-        float z = 1.f;
-        if constexpr (kGen) {
-          if (a.drop_thresh) z = drop_of(a, b, h, q0 + 8 * r4 + 4 * half + e, kvc);
+      rows_s[wave][lane] = row_val;
+      const bool finite_rows = __ballot(half == 0 && row_val == -INFINITY) == 0;
+      wave_order();
+      if (!seen_only && it + NW < items) fetch(it + NW);
+      float mb[16];
+      if constexpr (kGen) {
+        if (masked) {
+          mask_of_key(a, mb, (int64_t)b * a.msb + (int64_t)h * a.msh + (int64_t)kvc * a.msk, q0, half);
+          if (a.mask_kind == 1 && finite_rows && all_lanes_masked(mb)) continue;
         }
-        pz[r] = p * z;
-        dp[r] = p * fmaf(z, dp[r], -dl[e]);
       }
-    }
-    if (q0 + 32 > S || (!masked && qt == kb)) {
-      // queries past S, and (causal) the diagonal tile's queries before the key
-      const int from = masked ? 0 : kvrow;
+      f32x16_t s, dp;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int qr = q0 + 8 * (r >> 2) + 4 * half + (r & 3);
-        if (qr >= S || qr < from) {
-          pz[r] = 0.f;
-          dp[r] = 0.f;
+        s[r] = 0.f;
+        dp[r] = 0.f;
+      }
+      P::rows(cx, s, Qt, kf);
+      P::rows(cx, dp, Dt, vf);
+      f32x16_t pz;
+      uint32_t hidden = 0;
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        const float4 l4 = *reinterpret_cast<const float4*>(&rows_s[wave][8 * r4 + 4 * half]);
+        const float4 d4 = *reinterpret_cast<const float4*>(&rows_s[wave][32 + 8 * r4 + 4 * half]);
+        const float lv[4] = {l4.x, l4.y, l4.z, l4.w}, dl[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = 4 * r4 + e;
+          float x = s[r] * u;
+          if (masked) x = mb[r] == -INFINITY ? -INFINITY : x + mb[r];
+          const float p = exp_unit<P>(x - (P::kExact ? lv[e] : lv[e] * kLog2e));
+          float z = 1.f;
+          if constexpr (kGen) {
+            if (a.drop_thresh) z = drop_of(a, b, h, q0 + 8 * r4 + 4 * half + e, kvc);
+          }
+          pz[r] = p * z;
+          dp[r] = p * fmaf(z, dp[r], -dl[e]);
+          if constexpr (seen_only) {
+            const int qr = q0 + 8 * r4 + 4 * half + e;
+            hidden |= (qr >= S || (masked ? mb[r] == -INFINITY && lv[e] != -INFINITY : qr < kvrow)) ? 1u << r : 0u;
+          }
         }
       }
+      if (q0 + 32 > S || (!masked && qt == kb)) {
+        // queries past S, and (causal) the diagonal tile's queries before the key
+        const int from = masked ? 0 : kvrow;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int qr = q0 + 8 * (r >> 2) + 4 * half + (r & 3);
+          if (qr >= S || qr < from) {
+            pz[r] = 0.f;
+            dp[r] = 0.f;
+          }
+        }
+      }
+      if constexpr (seen_only) {
+        cols_seen<P>(dv, Dt, pz, hidden, lane);
+        cols_seen<P>(dk, Qt, dp, hidden, lane);
+      } else {
+        P::cols(cx, dv, Dt, pz);
+        P::cols(cx, dk, Qt, dp);
+      }
+      wave_order();
     }
-    P::cols(cx, dv, Dt, pz);
-    P::cols(cx, dk, Qt, dp);
-    wave_order();
+  };
+  pass(std::false_type{});
+  if constexpr (P::kExact) {
+    if (!all_finite(dk) || !all_finite(dv)) pass(std::true_type{});
   }
   wave_order();
   const bool valid = kvrow < S;
