@@ -8,7 +8,6 @@
 //           three may be column ranges of one fused QKV projection.
 //   o     : same row layout with H heads.
 //   lse   : [B, H, S] fp32, natural-log log-sum-exp of the scaled scores.
-//   *t    : transposed copies [B, heads, hd, S] (reduction index innermost).
 // The kv head of query head h is h / (H/KV); K/V are never expanded.
 //
 // MFMA tiling (v_mfma_f32_32x32x16_bf16).  The score tile is computed as
@@ -1385,9 +1384,13 @@ int tiles_bwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void
                                scale);
   wave_bwd_args(w, dout, lddo, delta, dq, lddq, dk, lddk, dv, lddv);
   w.delta_w = delta_w;
-  const bool can_wave = dtype == LZ_BF16 && lz_attn_wave_ok(w, dtype, hd, true);
-  const bool wave_dq = can_wave && wave_dq_better(S, lz_cdiv(S, 128) * B * H);
-  const bool wave_dkdv = can_wave && wave_dkdv_better(hd, S, lz_cdiv(S, 256) * B * KV);
+  // dout rows at 8 bytes (a slice of a flat gradient): at lengths the tiles do
+  // not divide they keep to kernels that load them through registers, as the
+  // direct-to-LDS copies are made for 16-byte rows
+  const bool dout8 = dtype == LZ_BF16 && S % 64 && !(lz_aligned16(dout) && lddo % 8 == 0);
+  const bool can_wave = dtype == LZ_BF16 && lz_attn_wave_ok(w, dtype, hd, true, dout8);
+  const bool wave_dq = can_wave && (dout8 || wave_dq_better(S, lz_cdiv(S, 128) * B * H));
+  const bool wave_dkdv = can_wave && (dout8 || wave_dkdv_better(hd, S, lz_cdiv(S, 256) * B * KV));
   rope_done = !wave_dq && !wave_dkdv;  // only the tile kernels rotate; the caller rotates after the others
   if (!rope_done) a.rcos = a.rsin = nullptr;
   // dQ first: it forms the delta that dK/dV reads when delta_w is set
@@ -1426,30 +1429,25 @@ int tiles_bwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void
 }  // namespace
 
 // What lz_attn_fwd/bwd take for these arguments: 2 = MFMA on LDS tiles (S a
-// multiple of 64; no transposed buffers), 1 = the same dtypes and head dims at
-// other lengths, for which lz_attn_fwd/bwd ask for transposed operand buffers
-// (V^T; Q^T, K^T, dO^T: required, no longer read) and lz_attn_fwd_direct /
-// lz_attn_bwd_direct do not, 0 = the rest.
+// multiple of 64), 1 = bf16 and the same head dims at other lengths, 0 = the
+// rest.
 LZ_EXPORT int lz_attn_path(int dtype, int64_t S, int64_t hd, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo) {
   const bool mfma = (dtype == LZ_BF16 || (dtype == LZ_F16 && S % 64 == 0)) && (hd == 64 || hd == 128) &&
                     strides_ok(ldq, ldk, ldv, ldo);
   return mfma ? (S % 64 == 0 ? 2 : 1) : 0;
 }
 
-// Forward.  vt: V^T [B,KV,hd,S] (required where lz_attn_path is 1).
+// Forward.  vt is ignored (no kernel reads a transposed operand).
 LZ_EXPORT int lz_attn_fwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
-                          const void* vt, void* o, int64_t ldo, float* lse, int64_t B, int64_t S, int64_t H, int64_t KV,
-                          int64_t hd, float scale, int dtype, void* stream) {
+                          const void* /*vt*/, void* o, int64_t ldo, float* lse, int64_t B, int64_t S, int64_t H,
+                          int64_t KV, int64_t hd, float scale, int dtype, void* stream) {
   int rc = check_shape(B, S, H, KV, hd);
   if (rc) return rc;
   LZ_REQUIRE(q && k && v && o && lse, "lz_attn_fwd: null pointer");
   hipStream_t s = lz_stream(stream);
   const bool mfma = mfma_ok(dtype, hd, ldq, ldk, ldv, ldo, q, k, v, o);
-  if (mfma && S % 64 == 0) return tiles_fwd(q, ldq, k, ldk, v, ldv, o, ldo, lse, B, S, H, KV, hd, scale, dtype, s);
-  if (mfma && dtype == LZ_BF16) {
-    LZ_REQUIRE(vt && lz_aligned16(vt), "lz_attn_fwd: this shape takes an aligned V^T buffer");
+  if (mfma && (dtype == LZ_BF16 || S % 64 == 0))
     return tiles_fwd(q, ldq, k, ldk, v, ldv, o, ldo, lse, B, S, H, KV, hd, scale, dtype, s);
-  }
   const LzWaveArgs w = wave_fwd_args(q, ldq, k, ldk, v, ldv, o, ldo, lse, B, S, H, KV, scale);
   if (lz_attn_wave_ok(w, dtype, hd, false)) return lz_attn_wave_pass(w, dtype, hd, kWaveSplit, kWaveFwd, s);
   const unsigned grid = (unsigned)lz_cdiv(B * H * S, 4);
@@ -1512,24 +1510,23 @@ LZ_EXPORT int lz_rope(void* x, int dtype, int64_t ld, int64_t rows, int64_t seq,
 namespace {
 
 int attn_bwd_impl(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, const void* dout,
-                  int64_t lddo, const float* lse, const float* delta, const void* qt, const void* kt, const void* dot,
-                  void* dq, int64_t lddq, void* dk, int64_t lddk, void* dv, int64_t lddv, int64_t B, int64_t S,
-                  int64_t H, int64_t KV, int64_t hd, float scale, const void* rope_cos, const void* rope_sin,
+                  int64_t lddo, const float* lse, const float* delta, void* dq, int64_t lddq, void* dk, int64_t lddk,
+                  void* dv, int64_t lddv, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t hd, float scale, const void* rope_cos, const void* rope_sin,
                   int dtype, hipStream_t s, bool& rope_done, const void* o = nullptr, int64_t ldo = 0,
                   float* delta_w = nullptr);
 
 }  // namespace
 
-// Backward.  Where lz_attn_path is 1 qt [B,H,hd,S], kt [B,KV,hd,S] and dot
-// [B,H,hd,S] are required; delta comes from lz_attn_delta.  dq/dk/dv are written (not
+// Backward.  qt, kt and dot are ignored (no kernel reads a transposed
+// operand); delta comes from lz_attn_delta.  dq/dk/dv are written (not
 // accumulated).  rope_cos/rope_sin (both or neither; tables [>= S, hd] in the
 // activation dtype, row = position, as lz_rope takes): dq and dk come back
 // as the gradients of q and k before RoPE, i.e. with lz_rope's backward
 // already applied (in the bf16 MFMA kernels' epilogue, otherwise by lz_rope
 // after them).
 LZ_EXPORT int lz_attn_bwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
-                          const void* dout, int64_t lddo, const float* lse, const float* delta, const void* qt,
-                          const void* kt, const void* dot, void* dq, int64_t lddq, void* dk, int64_t lddk, void* dv,
+                          const void* dout, int64_t lddo, const float* lse, const float* delta, const void* /*qt*/,
+                          const void* /*kt*/, const void* /*dot*/, void* dq, int64_t lddq, void* dk, int64_t lddk, void* dv,
                           int64_t lddv, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t hd, float scale,
                           const void* rope_cos, const void* rope_sin, int dtype, void* stream) {
   int rc = check_shape(B, S, H, KV, hd);
@@ -1541,8 +1538,8 @@ LZ_EXPORT int lz_attn_bwd(const void* q, int64_t ldq, const void* k, int64_t ldk
              "lz_attn_bwd: RoPE needs an even head dim and 8-byte aligned tables");
   hipStream_t s = lz_stream(stream);
   bool rope_done = false;
-  rc = attn_bwd_impl(q, ldq, k, ldk, v, ldv, dout, lddo, lse, delta, qt, kt, dot, dq, lddq, dk, lddk, dv, lddv, B, S,
-                     H, KV, hd, scale, rope_cos, rope_sin, dtype, s, rope_done);
+  rc = attn_bwd_impl(q, ldq, k, ldk, v, ldv, dout, lddo, lse, delta, dq, lddq, dk, lddk, dv, lddv, B, S, H, KV, hd,
+                     scale, rope_cos, rope_sin, dtype, s, rope_done);
   if (rc || rope_cos == nullptr || rope_done) return rc;
   rc = lz_rope(dq, dtype, lddq, B * S, S, H, hd, rope_cos, rope_sin, 0, 1, stream);
   if (rc) return rc;
@@ -1567,9 +1564,8 @@ LZ_EXPORT int lz_attn_bwd_with_o(const void* q, int64_t ldq, const void* k, int6
                                                         reinterpret_cast<uintptr_t>(rope_sin)) & 7) == 0),
              "lz_attn_bwd_with_o: RoPE needs an even head dim and 8-byte aligned tables");
   bool rope_done = false;
-  rc = attn_bwd_impl(q, ldq, k, ldk, v, ldv, dout, lddo, lse, delta, nullptr, nullptr, nullptr, dq, lddq, dk, lddk, dv,
-                     lddv, B, S, H, KV, hd, scale, rope_cos, rope_sin, dtype, lz_stream(stream), rope_done, o, ldo,
-                     delta);
+  rc = attn_bwd_impl(q, ldq, k, ldk, v, ldv, dout, lddo, lse, delta, dq, lddq, dk, lddk, dv, lddv, B, S, H, KV, hd,
+                     scale, rope_cos, rope_sin, dtype, lz_stream(stream), rope_done, o, ldo, delta);
   if (rc || rope_cos == nullptr || rope_done) return rc;
   rc = lz_rope(dq, dtype, lddq, B * S, S, H, hd, rope_cos, rope_sin, 0, 1, stream);
   if (rc) return rc;
@@ -1579,16 +1575,13 @@ LZ_EXPORT int lz_attn_bwd_with_o(const void* q, int64_t ldq, const void* k, int6
 namespace {
 
 int attn_bwd_impl(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, const void* dout,
-                  int64_t lddo, const float* lse, const float* delta, const void* qt, const void* kt, const void* dot,
-                  void* dq, int64_t lddq, void* dk, int64_t lddk, void* dv, int64_t lddv, int64_t B, int64_t S,
-                  int64_t H, int64_t KV, int64_t hd, float scale, const void* rope_cos, const void* rope_sin,
+                  int64_t lddo, const float* lse, const float* delta, void* dq, int64_t lddq, void* dk, int64_t lddk,
+                  void* dv, int64_t lddv, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t hd, float scale, const void* rope_cos, const void* rope_sin,
                   int dtype, hipStream_t s, bool& rope_done, const void* o, int64_t ldo, float* delta_w) {
   const bool mfma = mfma_ok(dtype, hd, ldq, ldk, ldv, lddo, q, k, v, dout) && lddq % 4 == 0 && lddk % 4 == 0 &&
                     lddv % 4 == 0;
   LZ_REQUIRE(delta_w == nullptr || (mfma && S % 64 == 0),
              "lz_attn_bwd_with_o: this shape takes the other kernels (use lz_attn_delta + lz_attn_bwd)");
-  LZ_REQUIRE(!(mfma && dtype == LZ_BF16 && S % 64) || (qt && kt && dot),
-             "lz_attn_bwd: this shape takes transposed Q, K and dO buffers");
   if (mfma && (dtype == LZ_BF16 || S % 64 == 0))
     return tiles_bwd(q, ldq, k, ldk, v, ldv, dout, lddo, lse, delta, dq, lddq, dk, lddk, dv, lddv, B, S, H, KV, hd,
                      scale, rope_cos, rope_sin, dtype, s, rope_done, o, ldo, delta_w);

@@ -35,8 +35,8 @@ struct LzWaveArgs {
 };
 
 // Whether these kernels take the call: head dim 32, 64 or 128, rows aligned
-// for their reads and writes.
-bool lz_attn_wave_ok(const LzWaveArgs& a, int dtype, int64_t hd, bool backward);
+// for their reads and writes (dout8: dout rows may start at any 8 bytes).
+bool lz_attn_wave_ok(const LzWaveArgs& a, int dtype, int64_t hd, bool backward, bool dout8 = false);
 
 // How a call is computed.  General: mask_kind and dropout are read (also when
 // both are off, so that a call with dropout has the lse of one without);

@@ -173,6 +173,14 @@ struct PolF32 {
   }
 };
 
+// 16 bytes from an 8-byte aligned address (the global loads of dout rows; one
+// instruction either way).
+typedef uint32_t u32x4a8_t __attribute__((ext_vector_type(4), aligned(8)));
+__device__ __forceinline__ uint4 load16(const uint16_t* p) {
+  const u32x4a8_t v = *reinterpret_cast<const u32x4a8_t*>(p);
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+
 template <int HD_, bool kSplit>
 struct PolBF16 {
   static constexpr int HD = HD_;
@@ -191,7 +199,7 @@ struct PolBF16 {
   static __device__ __forceinline__ void load_own(Own& f, const void* row, int half) {
 #pragma unroll
     for (int kk = 0; kk < HD / 16; ++kk)
-      f.x[kk] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(row) + 16 * kk + 8 * half));
+      f.x[kk] = __builtin_bit_cast(bf16x8_t, load16(static_cast<const uint16_t*>(row) + 16 * kk + 8 * half));
   }
   static __device__ __forceinline__ float dot(const Own& a, const Own& b) {
     float s = 0.f;
@@ -212,7 +220,7 @@ struct PolBF16 {
     for (int i = 0; i < kPieces; ++i) {
       const int p = lane + 64 * i;
       const int r = min(row0 + p / (HD / 8), S - 1);
-      st.p[i] = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(base) + r * ld + 8 * (p % (HD / 8)));
+      st.p[i] = load16(static_cast<const uint16_t*>(base) + r * ld + 8 * (p % (HD / 8)));
     }
   }
   static __device__ __forceinline__ void store(const Stage& st, char* tile, int row0, int S, int lane) {
@@ -879,7 +887,7 @@ int launch(const LzWaveArgs& a, LzWavePass pass, hipStream_t s) {
 
 }  // namespace
 
-bool lz_attn_wave_ok(const LzWaveArgs& a, int dtype, int64_t hd, bool backward) {
+bool lz_attn_wave_ok(const LzWaveArgs& a, int dtype, int64_t hd, bool backward, bool dout8) {
   if (hd != 32 && hd != 64 && hd != 128) return false;
   if (dtype != LZ_BF16 && dtype != LZ_F16 && dtype != LZ_F32) return false;
   if ((int64_t)a.B * a.H * ((a.S + 31) / 32) >= (1ll << 31)) return false;
@@ -891,7 +899,9 @@ bool lz_attn_wave_ok(const LzWaveArgs& a, int dtype, int64_t hd, bool backward) 
   auto writes = [&](const void* p, int64_t ld) { return (reinterpret_cast<uintptr_t>(p) & wr) == 0 && ld % 4 == 0; };
   if (!reads(a.q, a.ldq) || !reads(a.k, a.ldk) || !reads(a.v, a.ldv)) return false;
   if (!backward) return writes(a.o, a.ldo);
-  return reads(a.dout, a.lddo) && (a.delta_w == nullptr || reads(a.o, a.ldo)) && writes(a.dq, a.lddq) &&
+  const bool dout_ok = reads(a.dout, a.lddo) ||
+                       (dout8 && dtype != LZ_F32 && (reinterpret_cast<uintptr_t>(a.dout) & 7) == 0 && a.lddo % 4 == 0);
+  return dout_ok && (a.delta_w == nullptr || reads(a.o, a.ldo)) && writes(a.dq, a.lddq) &&
          writes(a.dk, a.lddk) && writes(a.dv, a.lddv);
 }
 

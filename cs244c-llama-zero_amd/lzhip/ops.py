@@ -998,10 +998,8 @@ def ce_bwd(logits2: torch.Tensor, labels: torch.Tensor, seq: int, lse: torch.Ten
 
 
 def attn_path(dtype: torch.dtype, S: int, hd: int, ldq: int, ldk: int, ldv: int, ldo: int) -> int:
-    """What attn_fwd/attn_bwd take: 2: MFMA on LDS tiles, 1: the same at other
-    lengths, where they ask for transposed operand buffers (V^T forward; Q^T,
-    K^T, dO^T backward) and attn_fwd_direct/attn_bwd_direct do not, 0: the
-    rest."""
+    """What attn_fwd/attn_bwd take: 2: MFMA on LDS tiles, 1: bf16 at other
+    lengths, 0: the rest."""
     if dtype not in _DTYPES:
         return 0
     return int(_lib.load().lz_attn_path(_DTYPES[dtype], S, hd, ldq, ldk, ldv, ldo))
@@ -1009,8 +1007,8 @@ def attn_path(dtype: torch.dtype, S: int, hd: int, ldq: int, ldk: int, ldv: int,
 
 def attn_fwd(q2: torch.Tensor, k2: torch.Tensor, v2: torch.Tensor, B: int, S: int, H: int, KV: int, hd: int,
              scale: float, vt: Optional[torch.Tensor]) -> Tuple[torch.Tensor, torch.Tensor]:
-    """q2/k2/v2: [B*S, ld] row views (head h at columns h*hd).  Returns
-    o [B*S, H*hd] and lse [B, H, S]."""
+    """q2/k2/v2: [B*S, ld] row views (head h at columns h*hd); vt is ignored.
+    Returns o [B*S, H*hd] and lse [B, H, S]."""
     require_gpu(q2, k2, v2, vt)
     o = torch.empty((B * S, H * hd), dtype=q2.dtype, device=q2.device)
     lse = torch.empty((B, H, S), dtype=torch.float32, device=q2.device)
@@ -1158,8 +1156,8 @@ def dropout_mask(n: int, p: float, seed: int, device: torch.device) -> torch.Ten
 
 def attn_bwd(q2, k2, v2, o2, do2, lse, B, S, H, KV, hd, scale, dq2, dk2, dv2, qt=None, kt=None, dot=None,
              rope: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> None:
-    """dq2/dk2/dv2 = gradients of causal GQA attention.  With rope = (cos,
-    sin) (rope_'s tables), dq2 and dk2 are the gradients of q and k before
+    """dq2/dk2/dv2 = gradients of causal GQA attention (qt, kt and dot are
+    ignored).  With rope = (cos, sin) (rope_'s tables), dq2 and dk2 are the gradients of q and k before
     RoPE: the RoPE backward is applied in the same call."""
     require_gpu(q2, k2, v2, o2, do2, lse, dq2, dk2, dv2)
     rc = rs = None

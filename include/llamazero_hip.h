@@ -301,11 +301,10 @@ int lz_gemm_swiglu_bwd(const void* dy, int64_t lddy, const void* w, int64_t ldw,
 /* Causal GQA flash attention (model/llama.py:88-117: repeat_kv +
  * F.scaled_dot_product_attention(is_causal=True)).  lz_attn_path reports what
  * lz_attn_fwd/bwd take: 2 = MFMA on LDS tiles (bf16 or fp16, hd 64 or 128, S a
- * multiple of 64; the transposed-operand arguments may be NULL), 1 = bf16 at
- * other lengths: vt (forward) and qt, kt, dot (backward, each [B, heads, hd,
- * S]) are required though no kernel reads them any more (the direct entry
- * points below take the same shapes without them), 0 = the rest (hd 32 and
- * fp32: wave-private MFMA kernels; other head dims: generic). */
+ * multiple of 64), 1 = bf16 at other lengths, 0 = the rest (hd 32 and fp32:
+ * wave-private MFMA kernels; other head dims: generic).  vt (forward) and qt,
+ * kt, dot (backward) are ignored and may be NULL: no kernel reads a transposed
+ * operand. */
 int lz_attn_path(int dtype, int64_t S, int64_t hd, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo);
 int lz_attn_fwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, const void* vt,
                 void* o, int64_t ldo, float* lse, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t hd, float scale,

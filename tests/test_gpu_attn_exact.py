@@ -157,3 +157,28 @@ def test_non_finite_rows_reach_only_what_sees_them(dtype, hd, kind, t, what):
         check("dk", dk, k.grad, kv_rows, gtol)
     if clean_kv["dv"]:
         check("dv", dv, v.grad, kv_rows, gtol)
+
+
+@pytest.mark.parametrize("S", [33, 200])
+@pytest.mark.parametrize("H,KV,hd", [(12, 4, 64), (16, 8, 128)])
+def test_output_gradient_at_an_8_byte_offset(H, KV, hd, S):
+    """The attention layer's backward takes an output gradient that is a slice
+    of a flat buffer (contiguous, 8- but not 16-byte aligned) at lengths that
+    are not a multiple of 64.
+    bf16 outputs of weights rounded once: the gradients differ from those of an
+    aligned copy by that rounding."""
+    from lzhip import functional as LF
+
+    B, d = 2, 256
+    g = torch.Generator(device=DEV).manual_seed(S + hd)
+    x = torch.randn(B, S, d, generator=g, device=DEV).to(BF16).requires_grad_()
+    w = [(0.06 * torch.randn(n * hd, d, generator=g, device=DEV)).to(BF16).requires_grad_() for n in (H, KV, KV)]
+    cos, sin = ops.rope_table(S, hd, 10000.0 ** (-torch.arange(0, hd, 2, device=DEV) / hd), BF16)
+    y = LF.AttnProjFn.apply(x, *w, cos, sin, H, KV, hd**-0.5)
+    flat = torch.randn(y.numel() + 4, generator=g, device=DEV).to(BF16)
+    do = flat[4:].view(y.shape)
+    assert do.data_ptr() % 16 == 8
+    got = torch.autograd.grad(y, [x, *w], do, retain_graph=True)
+    want = torch.autograd.grad(y, [x, *w], do.clone())
+    for a, b in zip(got, want):
+        assert float((a.double() - b.double()).norm() / b.double().norm()) < 1e-2
