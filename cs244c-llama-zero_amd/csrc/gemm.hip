@@ -1002,8 +1002,9 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, bool ak, bool bk) {
     const double old = p.cfg >= 5 ? plan_us(p.cfg, p.splits, M, N, K, bk, ak) : 1.8 * plan_us(5, p.splits, M, N, K, bk, ak);
     double best = 0.8 * old;
     // x.W^T of whole 256x256 tiles is what the fused SwiGLU and RoPE products
-    // compute too: unsplit, so that both give the same bits
-    const bool fused_too = ak && bk && M % 256 == 0 && N % 256 == 0;
+    // compute too, dy.W of them what SwiGLU's fused backward does: unsplit, so
+    // that both give the same bits (a dy.W of K >= 1024 may be split above)
+    const bool fused_too = ak && M % 256 == 0 && N % 256 == 0 && (bk || K < 1024);
     for (int cfg = 7; cfg <= 9; ++cfg) {
       for (int sp : {1, 2, 3, 4, 6, 8}) {
         if (sp > 1 && fused_too) break;

@@ -417,7 +417,8 @@ def test_gemm_swiglu_fused_matches_unfused(M, F_, K):
     assert float(diff.max()) <= 2 ** -6 * float(want.abs().max() + 1)
 
 
-@pytest.mark.parametrize("M,F_,K,pad", [(256, 256, 64, 0), (512, 768, 192, 8), (768, 512, 960, 0)])
+@pytest.mark.parametrize("M,F_,K,pad", [(256, 256, 64, 0), (512, 768, 192, 8), (768, 512, 960, 0), (256, 256, 832, 0),
+                                         (512, 256, 960, 0), (256, 512, 960, 8)])
 def test_gemm_swiglu_bwd_fused_matches_unfused(M, F_, K, pad):
     """The down projection's input gradient with SwiGLU's backward in its
     epilogue equals gemm (W_down read N-major) followed by the SwiGLU backward

@@ -429,6 +429,20 @@ def test_gemm_plan_codes_and_workspace():
     assert int(lib.lz_gemm_plan(0, 10, 10, 1, 1)) == 0
 
 
+def test_products_with_a_fused_twin_are_unsplit():
+    """x.W^T (fused SwiGLU, RoPE) and dy.W (SwiGLU's backward) of whole
+    256-tiles sum K < 1024 in one go, as the fused kernels do, so that fused
+    and unfused give the same bits."""
+    import lzhip._lib as L
+
+    if not L.LIB_PATH.exists():
+        pytest.skip("libllamazero_hip.so not built (run __graft_entry__.build())")
+    lib = L.load()
+    split = [(M, N, K, bk) for M in range(256, 2305, 256) for N in range(256, 4097, 256) for K in range(64, 1024, 64)
+             for bk in (0, 1) if int(lib.lz_gemm_plan(M, N, K, 1, bk)) % 64 != 1]
+    assert not split, split[:5]
+
+
 def test_loss_scaler_follows_torch_grad_scaler():
     """lzhip.optim.LossScaler's schedule (reference train.py:213-214,254-269:
     torch.cuda.amp.GradScaler) against torch.amp.GradScaler itself on the
