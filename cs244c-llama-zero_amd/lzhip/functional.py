@@ -426,6 +426,21 @@ class AttnProjFn(Function):
         return dh, dwq, dwk, dwv, None, None, None, None, None, None, None, None
 
 
+def down_wgrad_beside(d: int, ffn: int, tokens: int) -> bool:
+    """Whether W_down's gradient [d, ffn] over `tokens` rows runs on a second
+    stream beside the fused input gradient.  The events and the switch cost 70
+    us of host time, so the products have to be large, and only one that leaves
+    CUs idle or is bound by its output gains at all.  Whole backward of the MLP,
+    one stream / two (us): small tiles and split plans lose (125M 2048 tokens
+    96 / 139, 4096 138 / 153, 16384 in 8 slices 381 / 399; 1152 x 3072 4096 229 /
+    244); unsplit 256x256 tiles, 176 of them (2048 x 5632): 1024 tokens 193 / 196,
+    2048 296 / 306, 4096 572 / 576, 8192 1006 / 985, 16384 1954 / 1915; 688
+    of them (4096 x 11008): 512 tokens 375 / 355, 2048 992 / 960, 8192 3526 / 3560."""
+    if ops.gemm_plan(d, ffn, tokens, False, False) != (5, 1):
+        return False
+    return tokens >= 8192 or -(-d // 256) * -(-ffn // 256) >= ops.device_cus()
+
+
 class MLPFn(Function):
     """SwiGLU MLP (model/llama.py:136-146): down(silu(gate x) * up x), gate and
     up as one GEMM, with an optional residual added in the down projection's
@@ -472,16 +487,14 @@ class MLPFn(Function):
         if dropout_p == 0.0 and ops.swiglu_bwd_fusable(dy2, wd, gu):
             # dm = dy . W_down goes straight into SwiGLU's backward in the
             # GEMM's epilogue (same bits as the two kernels, dm never stored).
-            # An unsplit W_down gradient runs beside it on a second stream:
-            # that kernel's epilogue phases are HBM-bound with the matrix
-            # cores idle, the weight gradient's main loop is the opposite
-            # (1B shapes: 752 -> 709 us for the pair).  A split one (125M:
-            # 8 ways and a reduce) already fills the chip and measured no
-            # gain; other layers' input and weight gradients run slower
-            # side by side, so they do not.
+            # A large W_down gradient runs beside it on a second stream: that
+            # kernel's epilogue phases are HBM-bound with the matrix cores
+            # idle, the weight gradient's main loop is the opposite (1B
+            # shapes: 752 -> 709 us for the pair).  Other layers' input and
+            # weight gradients run slower side by side, so they do not.
             # (one stream while a graph is being captured)
             if (ctx.needs_input_grad[3] and not torch.cuda.is_current_stream_capturing()
-                    and ops.gemm_unsplit(wd.shape[0], wd.shape[1], dy2.shape[0], False, False)):
+                    and down_wgrad_beside(wd.shape[0], wd.shape[1], dy2.shape[0])):
                 main = torch.cuda.current_stream(dy2.device)
                 side = _side_stream(dy2.device)
                 side.wait_stream(main)

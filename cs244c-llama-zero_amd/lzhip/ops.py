@@ -647,9 +647,17 @@ class LaunchProbe:
         return {k: self.summary(k) for k in {r[3] for r in self.records}}
 
 
-def gemm_unsplit(M: int, N: int, K: int, a_kmajor: bool, b_kmajor: bool) -> bool:
-    """Whether lz_gemm runs this product without splitting K."""
-    return int(_lib.load().lz_gemm_plan(M, N, K, int(a_kmajor), int(b_kmajor))) % 64 == 1
+def device_cus() -> int:
+    """Compute units of the current device."""
+    return _lib.query("lz_device_cus")
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_plan(M: int, N: int, K: int, a_kmajor: bool, b_kmajor: bool) -> Tuple[int, int]:
+    """(tile configuration, K slices) of lz_gemm for this product; see
+    lz_gemm_plan."""
+    code = int(_lib.load().lz_gemm_plan(M, N, K, int(a_kmajor), int(b_kmajor)))
+    return code // 64, code % 64
 
 
 def gemm_kernel_name(key) -> str:

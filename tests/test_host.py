@@ -443,6 +443,20 @@ def test_products_with_a_fused_twin_are_unsplit():
     assert not split, split[:5]
 
 
+def test_which_down_projection_gradients_take_the_second_stream():
+    """Small-tile and split plans stay on one stream (they measured slower on
+    two), as do 256x256 plans too short to pay for the events."""
+    import lzhip._lib as L
+    from lzhip import functional as LF
+
+    if not L.LIB_PATH.exists():
+        pytest.skip("libllamazero_hip.so not built (run __graft_entry__.build())")
+    for d, ffn, tokens, beside in ((768, 2048, 256, False), (768, 2048, 2048, False), (768, 2048, 4096, False),
+                                   (768, 2048, 16384, False), (1152, 3072, 4096, False), (2048, 5632, 2048, False),
+                                   (2048, 5632, 8192, True), (2048, 5632, 16384, True), (4096, 11008, 512, True)):
+        assert LF.down_wgrad_beside(d, ffn, tokens) is beside, (d, ffn, tokens)
+
+
 def test_loss_scaler_follows_torch_grad_scaler():
     """lzhip.optim.LossScaler's schedule (reference train.py:213-214,254-269:
     torch.cuda.amp.GradScaler) against torch.amp.GradScaler itself on the
