@@ -134,7 +134,12 @@ class RotaryEmbedding(nn.Module):
         return self.cos_cached[:, :, :seq_len, :], self.sin_cached[:, :, :seq_len, :]
 
     def tables(self, seq_len: int, device: torch.device, dtype: torch.dtype) -> Tuple[torch.Tensor, torch.Tensor]:
-        """[S, hd] views of the cache for the fused kernels."""
+        """[S, hd] views of the cache for the fused kernels (of what forward()
+        returns where that is replaced)."""
+        forward = self.forward
+        if getattr(forward, "__func__", None) is not RotaryEmbedding.forward:
+            cos, sin = forward(seq_len, device, dtype)
+            return cos.reshape(-1, self.dim), sin.reshape(-1, self.dim)
         cos, sin = self.cos_cached, self.sin_cached
         if seq_len > self.max_seq_len_cached or cos.device != device or cos.dtype != dtype:
             self._build_cache(seq_len=seq_len, device=device, dtype=dtype)

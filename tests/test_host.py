@@ -457,6 +457,25 @@ def test_which_down_projection_gradients_take_the_second_stream():
         assert LF.down_wgrad_beside(d, ffn, tokens) is beside, (d, ffn, tokens)
 
 
+def test_rotary_tables_come_from_an_overridden_forward():
+    """A subclass (or an instance) that replaces RotaryEmbedding.forward, e.g.
+    to scale positions, is what the attention layer rotates by."""
+    from model.llama import RotaryEmbedding
+
+    class Scaled(RotaryEmbedding):
+        def forward(self, seq_len, device, dtype):
+            pos = torch.arange(seq_len, dtype=torch.float32)[:, None] * torch.ones(self.dim) / 4
+            return pos.cos()[None, None].to(dtype), pos.sin()[None, None].to(dtype)
+
+    want = (torch.arange(6, dtype=torch.float32)[:, None] * torch.ones(8) / 4)
+    rot = Scaled(8)
+    cos, sin = rot.tables(6, torch.device("cpu"), torch.float32)
+    assert torch.equal(cos, want.cos()) and torch.equal(sin, want.sin())
+    plain = RotaryEmbedding(8)
+    plain.forward = rot.forward
+    assert torch.equal(plain.tables(6, torch.device("cpu"), torch.float32)[0], want.cos())
+
+
 def test_loss_scaler_follows_torch_grad_scaler():
     """lzhip.optim.LossScaler's schedule (reference train.py:213-214,254-269:
     torch.cuda.amp.GradScaler) against torch.amp.GradScaler itself on the
