@@ -17,7 +17,7 @@ import torch
 from . import _lib
 from ._lib import BF16, F16, F32
 
-_raw_stream = torch._C._cuda_getCurrentRawStream
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # torch builds with a GPU backend have it
 _DTYPES = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16}
 # 16-bit float formats (the MFMA GEMM and attention operands)
 HALF_DTYPES = (torch.bfloat16, torch.float16)

@@ -6,6 +6,8 @@ from __future__ import annotations
 
 import ctypes
 import re
+import subprocess
+import sys
 import time
 from pathlib import Path
 
@@ -474,6 +476,15 @@ def test_rotary_tables_come_from_an_overridden_forward():
     plain = RotaryEmbedding(8)
     plain.forward = rot.forward
     assert torch.equal(plain.tables(6, torch.device("cpu"), torch.float32)[0], want.cos())
+
+
+def test_package_imports_where_torch_has_no_gpu_symbols():
+    """A torch build without a GPU backend (tooling, CPU multi-process runs)
+    lacks torch._C's stream getter; importing the package must not need it."""
+    code = ("import torch; del torch._C._cuda_getCurrentRawStream\n"
+            "import lzhip, model, zero\nfrom lzhip import ops\nprint('imported')")
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT / "cs244c-llama-zero_amd")
+    assert out.stdout.strip() == "imported", out.stderr[-500:]
 
 
 def test_loss_scaler_follows_torch_grad_scaler():
