@@ -26,7 +26,7 @@ CSRC = Path(__file__).resolve().parent.parent / "cs244c-llama-zero_amd" / "csrc"
 sys.path.insert(0, str(CSRC))
 import build as B  # noqa: E402  (csrc/build.py: the library's compiler flags)
 
-SOURCES = ["gemm.hip", "attn.hip"]  # the sources that call lz_dma16
+SOURCES = [s for s in B.SOURCES if "lz_dma" in (CSRC / s).read_text()]  # the sources that issue such loads
 WAIT_STATES = 5
 
 
@@ -119,6 +119,8 @@ def test_direct_to_lds_loads_have_their_wait_states():
         total = 0
         for s in SOURCES:
             loads, found = hazards(outs[s].read_text())
+            assert loads > 0, s
             assert not found, f"{s}: {found[:3]}"
             total += loads
+    assert {"gemm.hip", "gemm_pipe.hip", "attn.hip"} <= set(SOURCES)
     assert total > 0  # the scan saw the loads it is meant to check
