@@ -19,6 +19,9 @@
 // group and the query blocks at or after the diagonal) and a dQ pass (one
 // workgroup per 128 queries, looping over key blocks up to the diagonal); no
 // atomics, deterministic.
+#include <algorithm>
+#include <cmath>
+
 #include "attn_tiles.h"
 #include "attn_wave.h"
 
@@ -1299,26 +1302,40 @@ void wave_bwd_args(LzWaveArgs& a, const void* dout, int64_t lddo, const float* d
 
 // Where the tile kernels' workgroups are too few to fill the chip the
 // wave-private kernels (a quarter or an eighth of the rows per workgroup, the
-// other side split over its waves) are faster; `wgs` is the tile kernel's
-// grid.  Lines drawn from both sides at B 1..8, S 128..2048, heads 12/4 and
-// 32/8 of 64 and 16/8 of 128 (us, tile / wave):
-//   forward, hd 64: 96 workgroups S 1024 16.1 / 11.5, S 512 10.0 / 8.8,
-//     S 256 7.0 / 7.6; 192 at S 2048 28.4 / 26.8, S 1024 16.7 / 18.4; hd 128: 64
-//     at S 512 13.8 / 12.0, 112 at S 777 19.7 / 19.1, 128 at S 1024 24.1 / 25.0
-//   dQ gains 1-5 us up to 64 workgroups, and at 96-128 where S >= 768
-//   dK/dV (256 keys and every query head of the group per tile workgroup):
-//     hd 64: 32 workgroups 109 / 43 for the whole backward, 192 at S 1536
-//     194 / 181, 256 at S 1024 204 / 226; hd 128: 64 at S 1024 134 / 82, 128 at
-//     S 2048 260 / 235 and S 777 144 / 101, at S 512 86 / 91
+// other side split over its waves) are faster.  A tile kernel's time is one
+// workgroup's chain of steps until its workgroups (`wgs`) fill the CUs; the
+// wave kernels cut that chain and grow with the work.  So the line is a share
+// of the CUs that rises with the steps of the chain: 64-key steps for the
+// forward and dQ, for dK/dV the 64-query steps over every query head of the
+// group, against its 32-key blocks in units of a tile workgroup's eight.
+// Lines from both sides over B 1..32, S 32..2048 (whole and ragged), heads 12/4,
+// 32/8, 8/8 of 64 and 16/8, 32/8, 32/32 of 128: over those 205 calls the rules
+// are within 0.1-0.3 % of the faster kernel in the geometric mean.  us, tile /
+// wave:
+//   forward, hd 64: 96 workgroups S 256 6.5 / 8.0, S 512 9.7 / 8.6, 192 S 1024
+//     16.1 / 18.2, S 2048 27.9 / 26.7; hd 128: 64 S 192 7.0 / 8.5, S 512 13.2 / 11.4,
+//     112 S 777 19.1 / 18.6, 128 S 1024 22.7 / 24.2
+//   dQ, hd 64: 48 S 64 5.5 / 6.9, 96 S 512 11.3 / 13.9, S 1024 17.4 / 14.7, 192 S 2048
+//     29.9 / 31.3; hd 128: 96 S 333 15.1 / 16.6, 112 S 777 25.1 / 22.5
+//   dK/dV, hd 64, heads 8/8: 128 workgroups S 512 21.2 / 24.6, S 1024 35.5 / 31.9; heads
+//     32/8: 128 S 2048 243 / 122, 256 S 2048 236 / 238; hd 128, heads 32/32: 64 S 256
+//     23.6 / 18.3, 128 S 512 36.4 / 44.6, S 500 45.9 / 45.0; heads 16/8: 128 S 512 57.8 /
+//     62.9, S 2048 193 / 169; heads of 128 at ragged lengths spill in the tile
+//     kernel (16/8, S 777: 110 / 69)
 bool wave_fwd_better(int64_t hd, int64_t S, int64_t wgs) {
-  if (wgs <= 64) return true;
-  if (hd == 64) return (wgs <= 96 && S > 256) || (wgs <= 192 && S > 1024);
-  return wgs <= 112 && S >= 768;
+  const double steps = (double)lz_cdiv(S, 64), share = (double)wgs / lz_num_cus();
+  if (hd == 64) return steps >= 2 && share <= std::max(0.28, 0.9 - 2.5 / steps);
+  return steps >= 4 && share <= 0.525 - 1.05 / steps;
 }
-bool wave_dq_better(int64_t S, int64_t wgs) { return wgs <= 64 || (wgs <= 128 && S >= 768); }
-bool wave_dkdv_better(int64_t hd, int64_t S, int64_t wgs) {
-  if (hd == 64) return wgs <= 192;
-  return wgs < 128 || (wgs == 128 && (S > 512 || S % 64));
+bool wave_dq_better(int64_t S, int64_t wgs) {
+  const double steps = (double)lz_cdiv(S, 64), share = (double)wgs / lz_num_cus();
+  return steps >= 2 && share <= std::min(0.21 + 0.02 * steps, 0.55);
+}
+bool wave_dkdv_better(int64_t hd, int64_t S, int64_t pairs, int64_t rep) {  // pairs: B * KV
+  const double cus = lz_num_cus(), steps = std::log2((double)(rep * lz_cdiv(S, 64)));
+  if (pairs * lz_cdiv(S, 256) >= cus) return false;
+  const double line = hd == 64 ? 0.04 + 0.12 * steps : (0.14 + 0.072 * steps) * (S % 64 ? 1.5 : 1.0);
+  return pairs * lz_cdiv(S, 32) / 8.0 <= cus * std::max(0.125, line);
 }
 
 // The forward of 16-bit causal attention with head dim 64 or 128 (aligned as
@@ -1390,7 +1407,7 @@ int tiles_bwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void
   const bool dout8 = dtype == LZ_BF16 && S % 64 && !(lz_aligned16(dout) && lddo % 8 == 0);
   const bool can_wave = dtype == LZ_BF16 && lz_attn_wave_ok(w, dtype, hd, true, dout8);
   const bool wave_dq = can_wave && (dout8 || wave_dq_better(S, lz_cdiv(S, 128) * B * H));
-  const bool wave_dkdv = can_wave && (dout8 || wave_dkdv_better(hd, S, lz_cdiv(S, 256) * B * KV));
+  const bool wave_dkdv = can_wave && (dout8 || wave_dkdv_better(hd, S, B * KV, H / KV));
   rope_done = !wave_dq && !wave_dkdv;  // only the tile kernels rotate; the caller rotates after the others
   if (!rope_done) a.rcos = a.rsin = nullptr;
   // dQ first: it forms the delta that dK/dV reads when delta_w is set
@@ -1435,6 +1452,18 @@ LZ_EXPORT int lz_attn_path(int dtype, int64_t S, int64_t hd, int64_t ldq, int64_
   const bool mfma = (dtype == LZ_BF16 || (dtype == LZ_F16 && S % 64 == 0)) && (hd == 64 || hd == 128) &&
                     strides_ok(ldq, ldk, ldv, ldo);
   return mfma ? (S % 64 == 0 ? 2 : 1) : 0;
+}
+
+// Which passes of causal attention on 16-byte aligned rows the tile kernels
+// run: 1 forward, 2 dQ, 4 dK/dV (the others are wave-private or generic).
+// Host only: attributes timings, and tests assert what they reach.
+LZ_EXPORT int lz_attn_tiles(int dtype, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t hd) {
+  if (B <= 0 || S <= 0 || KV <= 0 || H <= 0 || H % KV || (hd != 64 && hd != 128)) return 0;
+  if (dtype == LZ_F16) return S % 64 ? 0 : 7;
+  if (dtype != LZ_BF16) return 0;
+  const int64_t wgs = lz_cdiv(S, 128) * B * H;
+  return (wave_fwd_better(hd, S, wgs) ? 0 : 1) | (wave_dq_better(S, wgs) ? 0 : 2) |
+         (wave_dkdv_better(hd, S, B * KV, H / KV) ? 0 : 4);
 }
 
 // Forward.  vt is ignored (no kernel reads a transposed operand).

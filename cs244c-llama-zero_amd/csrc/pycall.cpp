@@ -122,6 +122,7 @@ Slot kSlots[] = {
     LZ_ENTRY(lz_gemm_workspace),
     LZ_ENTRY(lz_gemm_plan),
     LZ_ENTRY(lz_attn_path),
+    LZ_ENTRY(lz_attn_tiles),
     LZ_ENTRY(lz_attn_fwd),
     LZ_ENTRY(lz_attn_delta),
     LZ_ENTRY(lz_attn_fwd_general),

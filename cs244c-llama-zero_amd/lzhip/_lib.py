@@ -86,6 +86,7 @@ SIGNATURES = {
     "lz_gemm_workspace": (_i64, [_i64, _i64, _i64, _i32, _i32]),
     "lz_gemm_plan": (_i32, [_i64, _i64, _i64, _i32, _i32]),
     "lz_attn_path": (_i32, [_i32, _i64, _i64, _i64, _i64, _i64, _i64]),
+    "lz_attn_tiles": (_i32, [_i32, _i64, _i64, _i64, _i64, _i64]),
     "lz_attn_fwd": (
         _i32,
         [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _f32, _i32, _vp],

@@ -1013,6 +1013,12 @@ def attn_path(dtype: torch.dtype, S: int, hd: int, ldq: int, ldk: int, ldv: int,
     return int(_lib.load().lz_attn_path(_DTYPES[dtype], S, hd, ldq, ldk, ldv, ldo))
 
 
+def attn_tiles(dtype: torch.dtype, B: int, S: int, H: int, KV: int, hd: int) -> int:
+    """Which passes of causal attention the LDS-tile kernels run on aligned
+    rows: 1 forward, 2 dQ, 4 dK/dV."""
+    return int(_lib.load().lz_attn_tiles(_DTYPES[dtype], B, S, H, KV, hd))
+
+
 def attn_fwd(q2: torch.Tensor, k2: torch.Tensor, v2: torch.Tensor, B: int, S: int, H: int, KV: int, hd: int,
              scale: float, vt: Optional[torch.Tensor]) -> Tuple[torch.Tensor, torch.Tensor]:
     """q2/k2/v2: [B*S, ld] row views (head h at columns h*hd); vt is ignored.

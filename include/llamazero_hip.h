@@ -306,6 +306,10 @@ int lz_gemm_swiglu_bwd(const void* dy, int64_t lddy, const void* w, int64_t ldw,
  * kt, dot (backward) are ignored and may be NULL: no kernel reads a transposed
  * operand. */
 int lz_attn_path(int dtype, int64_t S, int64_t hd, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo);
+/* Which passes of causal attention on 16-byte aligned rows run on the LDS-tile
+ * kernels (1 forward, 2 dQ, 4 dK/dV; the others on the wave-private ones).
+ * Diagnostic only; no reference counterpart. */
+int lz_attn_tiles(int dtype, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t hd);
 int lz_attn_fwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, const void* vt,
                 void* o, int64_t ldo, float* lse, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t hd, float scale,
                 int dtype, void* stream);

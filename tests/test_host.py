@@ -431,6 +431,48 @@ def test_gemm_plan_codes_and_workspace():
     assert int(lib.lz_gemm_plan(0, 10, 10, 1, 1)) == 0
 
 
+def test_attention_kernel_rules_have_one_line_each():
+    """Which passes of bf16 causal attention run on the tile kernels: with more
+    sequences a pass moves to them once and stays; the benchmarks' shapes run
+    on them whole, a short prompt's on the wave-private kernels."""
+    import lzhip._lib as L
+    from lzhip import ops
+
+    if not L.LIB_PATH.exists():
+        pytest.skip("libllamazero_hip.so not built (run __graft_entry__.build())")
+    for H, KV, hd in ((12, 4, 64), (32, 8, 64), (8, 8, 64), (16, 8, 128), (32, 32, 128)):
+        for S in (1, 33, 64, 100, 128, 192, 256, 333, 512, 777, 1000, 1024, 2048, 4096):
+            codes = [ops.attn_tiles(torch.bfloat16, B, S, H, KV, hd) for B in range(1, 300)]
+            for bit in (1, 2, 4):
+                assert sorted(c & bit for c in codes) == [c & bit for c in codes], (H, KV, hd, S, bit)
+            assert codes[-1] == 7
+    assert ops.attn_tiles(torch.bfloat16, 16, 1024, 12, 4, 64) == 7
+    assert ops.attn_tiles(torch.bfloat16, 8, 2048, 16, 8, 128) == 7
+    assert ops.attn_tiles(torch.bfloat16, 1, 333, 12, 4, 64) == 0
+    assert ops.attn_tiles(torch.float16, 1, 320, 12, 4, 64) == 7 and ops.attn_tiles(torch.float16, 64, 333, 12, 4, 64) == 0
+    assert ops.attn_tiles(torch.float32, 64, 512, 12, 4, 64) == 0 and ops.attn_tiles(torch.bfloat16, 64, 512, 12, 4, 32) == 0
+
+
+def test_direct_attention_rule_matches_the_library():
+    """ops.attn_direct restates lz_attn_direct (and the pointers' alignment)
+    without the call: the same answer for every type, head dim and stride."""
+    import lzhip._lib as L
+    from lzhip import ops
+
+    if not L.LIB_PATH.exists():
+        pytest.skip("libllamazero_hip.so not built (run __graft_entry__.build())")
+    lib = L.load()
+    for dtype in (torch.bfloat16, torch.float16, torch.float32):
+        for hd in (16, 32, 48, 64, 128, 256):
+            for pad in range(9):
+                t = torch.empty(4 * (3 * hd + pad), dtype=dtype)[: 3 * (3 * hd + pad)].view(3, -1)
+                assert t.data_ptr() % 16 == 0
+                ld = t.stride(0)
+                want = bool(lib.lz_attn_direct(ops._DTYPES[dtype], hd, ld, ld, ld, ld))
+                assert ops.attn_direct(t, t, t, hd) is want, (dtype, hd, ld)
+            assert not ops.attn_direct(t[:, 1:], t, t, hd)
+
+
 def test_products_with_a_fused_twin_are_unsplit():
     """x.W^T (fused SwiGLU, RoPE) and dy.W (SwiGLU's backward) of whole
     256-tiles sum K < 1024 in one go, as the fused kernels do, so that fused
