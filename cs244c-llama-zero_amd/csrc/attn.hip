@@ -1309,9 +1309,9 @@ void wave_bwd_args(LzWaveArgs& a, const void* dout, int64_t lddo, const float* d
 // forward and dQ, for dK/dV the 64-query steps over every query head of the
 // group, against its 32-key blocks in units of a tile workgroup's eight.
 // Lines from both sides over B 1..32, S 32..2048 (whole and ragged), heads 12/4,
-// 32/8, 8/8 of 64 and 16/8, 32/8, 32/32 of 128: over those 205 calls the rules
-// are within 0.1-0.3 % of the faster kernel in the geometric mean.  us, tile /
-// wave:
+// 32/8, 8/8 of 64 and 16/8, 32/8, 32/32 of 128: over those 244 calls the rules
+// are within 0.1 % (forward), 0.4 % (dQ) and 0.5 % (dK/dV) of the faster kernel
+// in the geometric mean.  us, tile / wave:
 //   forward, hd 64: 96 workgroups S 256 6.5 / 8.0, S 512 9.7 / 8.6, 192 S 1024
 //     16.1 / 18.2, S 2048 27.9 / 26.7; hd 128: 64 S 192 7.0 / 8.5, S 512 13.2 / 11.4,
 //     112 S 777 19.1 / 18.6, 128 S 1024 22.7 / 24.2

@@ -243,22 +243,24 @@ def test_gemm_and_attention_repeat_bit_identically():
         first = fn().cpu()
         for _ in range(8):
             assert torch.equal(fn().cpu(), first), name
-    B, S, H, KV, hd = 2, 1024, 8, 4, 128
-    ld = (H + 2 * KV) * hd
-    d = torch.randn(B * S, ld, generator=g).to(torch.bfloat16).to(DEV)
-    q2, k2, v2 = d[:, : H * hd], d[:, H * hd : (H + KV) * hd], d[:, (H + KV) * hd :]
-    do = torch.randn(B * S, H * hd, generator=g).to(torch.bfloat16).to(DEV)
-    o0, lse0 = ops.attn_fwd(q2, k2, v2, B, S, H, KV, hd, hd**-0.5, None)
-    grads0 = None
-    for _ in range(6):
-        o, lse = ops.attn_fwd(q2, k2, v2, B, S, H, KV, hd, hd**-0.5, None)
-        assert torch.equal(o, o0) and torch.equal(lse, lse0)
-        dqkv = torch.zeros_like(d)
-        ops.attn_bwd(q2, k2, v2, o, do, lse, B, S, H, KV, hd, hd**-0.5, dqkv[:, : H * hd],
-                     dqkv[:, H * hd : (H + KV) * hd], dqkv[:, (H + KV) * hd :])
-        if grads0 is None:
-            grads0 = dqkv.cpu()
-        assert torch.equal(dqkv.cpu(), grads0)
+    for B, S, H, KV, hd, tiles in ((2, 1024, 8, 4, 128, 0), (16, 1024, 16, 8, 128, 7), (16, 1000, 16, 8, 128, 7),
+                                   (16, 1024, 12, 4, 64, 7)):
+        assert ops.attn_tiles(torch.bfloat16, B, S, H, KV, hd) & 6 == tiles & 6
+        ld = (H + 2 * KV) * hd
+        d = torch.randn(B * S, ld, generator=g).to(torch.bfloat16).to(DEV)
+        q2, k2, v2 = d[:, : H * hd], d[:, H * hd : (H + KV) * hd], d[:, (H + KV) * hd :]
+        do = torch.randn(B * S, H * hd, generator=g).to(torch.bfloat16).to(DEV)
+        o0, lse0 = ops.attn_fwd(q2, k2, v2, B, S, H, KV, hd, hd**-0.5, None)
+        grads0 = None
+        for _ in range(6):
+            o, lse = ops.attn_fwd(q2, k2, v2, B, S, H, KV, hd, hd**-0.5, None)
+            assert torch.equal(o, o0) and torch.equal(lse, lse0)
+            dqkv = torch.zeros_like(d)
+            ops.attn_bwd(q2, k2, v2, o, do, lse, B, S, H, KV, hd, hd**-0.5, dqkv[:, : H * hd],
+                         dqkv[:, H * hd : (H + KV) * hd], dqkv[:, (H + KV) * hd :])
+            if grads0 is None:
+                grads0 = dqkv.clone()
+            assert torch.equal(dqkv, grads0)
 
 
 def test_gemm_unaligned_mn_major_operands_fall_back():
@@ -718,12 +720,16 @@ def test_attention_dropout_vs_oracle(mask_kind, B, S, H, KV, hd, dtype, p):
 
 @pytest.mark.parametrize("B,S,H,KV,hd,dtype", [(2, 256, 8, 4, 128, torch.bfloat16), (1, 128, 4, 2, 64, torch.bfloat16),
                                                (1, 200, 4, 2, 128, torch.bfloat16), (2, 64, 4, 2, 32, torch.bfloat16),
-                                               (1, 96, 4, 2, 64, torch.float32)])
+                                               (1, 96, 4, 2, 64, torch.float32),
+                                               # large enough for the tile kernels in every pass
+                                               (32, 320, 16, 8, 128, torch.bfloat16), (32, 320, 12, 4, 64, torch.bfloat16),
+                                               (32, 289, 16, 8, 128, torch.bfloat16), (64, 289, 12, 4, 64, torch.bfloat16)])
 def test_attention_bwd_with_rope_equals_separate_rope(B, S, H, KV, hd, dtype):
     """attn_bwd(rope=(cos, sin)) returns exactly what attn_bwd followed by
-    the RoPE backward pass on dq and dk returns, on every kernel path (the
-    bf16 tile and transposed-operand paths fold the rotation into their
-    stores; the others run the RoPE kernel after)."""
+    the RoPE backward pass on dq and dk returns, on every kernel path (where
+    the tile kernels run dQ and dK/dV they fold the rotation into their
+    stores; otherwise the RoPE kernel runs after)."""
+    assert ops.attn_tiles(dtype, B, S, H, KV, hd) == (7 if B >= 32 else 0)
     g = _seed(B * S * hd + H)
     ld = (H + 2 * KV) * hd
     d = torch.randn(B * S, ld, generator=g).to(dtype).to(DEV)
@@ -771,7 +777,9 @@ def test_attention_delta(B, S, H, hd, pad):
 
 
 @pytest.mark.parametrize("B,S,H,KV,hd,dtype", [(2, 256, 4, 2, 128, torch.bfloat16), (1, 192, 6, 2, 64, torch.bfloat16),
-                                               (1, 128, 4, 4, 64, torch.float16), (1, 320, 4, 2, 128, torch.bfloat16)])
+                                               (1, 128, 4, 4, 64, torch.float16), (1, 320, 4, 2, 128, torch.bfloat16),
+                                               # large enough for the tile kernels in every pass
+                                               (32, 320, 16, 8, 128, torch.bfloat16), (32, 320, 12, 4, 64, torch.bfloat16)])
 def test_attention_bwd_with_o_matches_separate_delta(B, S, H, KV, hd, dtype):
     """lz_attn_bwd_with_o (delta computed by the dQ kernel, which then runs
     before dK/dV) against lz_attn_delta + lz_attn_bwd on the same inputs:
@@ -779,6 +787,7 @@ def test_attention_bwd_with_o_matches_separate_delta(B, S, H, KV, hd, dtype):
     order) and dq/dk/dv to the 16-bit format's rounding of that difference;
     with RoPE tables both return the pre-RoPE gradients.  S = 320 leaves the
     last 128-query block half outside the sequence."""
+    assert ops.attn_tiles(dtype, B, S, H, KV, hd) == (7 if B >= 32 or dtype == torch.float16 else 0)
     g = _seed(B * S * H + hd)
     ld = (H + 2 * KV) * hd
     qkv = torch.randn(B * S, ld, generator=g).to(dtype).to(DEV)
@@ -1191,13 +1200,17 @@ def test_copy2d_exact(dtype):
                                            (2, 63, 4, 2, "bool"), (2, 130, 4, 1, "bool"), (1, 97, 2, 2, "lowest"),
                                            (1, 96, 4, 2, "strided"), (1, 40, 2, 1, "dropout")])
 def test_attention_wave_private_kernels(B, S, H, KV, kind, hd, dtype):
-    """The wave-private kernels (and the ragged tile kernels: S 600 of bf16
-    heads of 64 and 128) at the edges of their 32- and 64-row tiles, against
-    float64: causal, bool masks with a query that sees nothing (NaN there and
+    """The wave-private kernels (causal bf16 heads of 64 and 128 take the tile
+    kernels' forward and dQ at a few dozen tokens) at the edges of their 32-row
+    tiles, against float64: causal, bool masks with a query that sees nothing (NaN there and
     only there) and keys nobody sees (their V may hold inf), additive masks
     of the type's lowest value and of arbitrary strides, and dropout.
     Tolerances: one rounding of the output type (bf16 2^-9, fp16 2^-12 per
     value) of intermediate P or O, fp32 sums 1e-5, as the tests above."""
+    tiles = 0
+    if dtype == torch.bfloat16 and hd > 32:
+        tiles = (1 if S <= (64 if hd == 64 else 192) else 0) | (2 if S <= 64 else 0)
+    assert kind is not None or ops.attn_tiles(dtype, B, S, H, KV, hd) == tiles
     g = _seed(B * S + hd + len(kind or ""))
     ld = (H + 2 * KV) * hd
     qkv = torch.randn(B * S, ld, generator=g).to(dtype)
@@ -1324,3 +1337,61 @@ def test_gemm_weight_gradient_k_tail(M, N, K, dtype):
     tol = 1e-5 * math.sqrt(K) * float(a[:K].float().abs().max() * b[:K].float().abs().max()) * 4
     assert float((c.double() - ref).abs().max()) <= tol
     assert torch.equal(ops.gemm(a[:K], b[:K], False, False), c.to(dtype))
+
+
+@pytest.mark.parametrize("B,S,H,KV,hd", [
+    # whole blocks
+    (32, 320, 12, 4, 64), (8, 1024, 32, 8, 64), (32, 256, 16, 8, 128),
+    # 1, 31, 33 and 63 rows past a 64-row block; one, two and three 256-key blocks; one to four query heads a group
+    (64, 33, 12, 4, 64), (64, 95, 8, 8, 64), (64, 129, 16, 4, 64), (32, 287, 12, 4, 64), (32, 289, 32, 8, 64),
+    (32, 321, 8, 8, 64), (32, 511, 12, 4, 64), (32, 543, 12, 4, 64), (64, 63, 32, 8, 128), (64, 65, 16, 8, 128),
+    (32, 287, 16, 8, 128), (32, 289, 16, 8, 128), (32, 321, 8, 8, 128), (16, 511, 32, 16, 128), (16, 577, 16, 16, 128)])
+def test_attention_tile_kernels(B, S, H, KV, hd):
+    """bf16 causal attention on grids that run every pass on the tile kernels
+    (their ragged instances where S is not a multiple of 64: clamped tails,
+    4-byte lse and delta copies, a last query block of fewer rows), against
+    float64: o within 1e-2 and the gradients within 2e-2 (weights and outputs
+    rounded to bf16), lse within 1e-3 (scores of bf16 products in fp32).  The
+    rows after the last sequence hold NaN: nothing past the end is read into a
+    result."""
+    assert ops.attn_tiles(torch.bfloat16, B, S, H, KV, hd) == 7
+    g = torch.Generator(device=DEV).manual_seed(B * S + hd)
+    ld = (H + 2 * KV) * hd
+    buf = torch.full((B * S + 64, ld), float("nan"), device=DEV, dtype=torch.bfloat16)
+    d = buf[: B * S]
+    d.copy_(torch.randn(B * S, ld, generator=g, device=DEV))
+    dobuf = torch.full((B * S + 64, H * hd), float("nan"), device=DEV, dtype=torch.bfloat16)
+    do = dobuf[: B * S]
+    do.copy_(torch.randn(B * S, H * hd, generator=g, device=DEV))
+    q2, k2, v2 = d[:, : H * hd], d[:, H * hd : (H + KV) * hd], d[:, (H + KV) * hd :]
+    scale = hd**-0.5
+    o, lse = ops.attn_fwd_direct(q2, k2, v2, B, S, H, KV, hd, scale)
+    grads = torch.full((B * S + 8, ld), 7.0, device=DEV, dtype=torch.bfloat16)
+    dq, dk, dv = (t[: B * S] for t in (grads[:, : H * hd], grads[:, H * hd : (H + KV) * hd], grads[:, (H + KV) * hd :]))
+    ops.attn_bwd_direct(q2, k2, v2, o, do, lse, B, S, H, KV, hd, scale, dq, dk, dv)
+    assert bool((grads[B * S :] == 7.0).all())
+    hidden = torch.ones(S, S, dtype=torch.bool, device=DEV).triu(1)
+    err = {}
+    num, den = {}, {}
+    for b in range(B):  # one sequence at a time: float64 scores of all of them would be gigabytes
+        rows = slice(b * S, (b + 1) * S)
+        heads = lambda t, n: t[rows].double().view(S, n, hd).transpose(0, 1)  # noqa: E731
+        q, k, v, dO = heads(q2, H), heads(k2, KV), heads(v2, KV), heads(do, H)
+        K, V = k.repeat_interleave(H // KV, 0), v.repeat_interleave(H // KV, 0)
+        s = (torch.matmul(q, K.transpose(1, 2).contiguous()) * scale).masked_fill(hidden, -math.inf)
+        P = torch.softmax(s, -1)
+        O = torch.matmul(P, V)
+        dP = torch.matmul(dO, V.transpose(1, 2).contiguous())
+        dS = P * (dP - (dO * O).sum(-1, keepdim=True))
+        grp = lambda t: t.view(KV, H // KV, S, hd).sum(1)  # noqa: E731
+        ref = {"o": (o, O, H), "dq": (dq, scale * torch.matmul(dS, K), H),
+               "dk": (dk, grp(scale * torch.matmul(dS.transpose(1, 2).contiguous(), q)), KV),
+               "dv": (dv, grp(torch.matmul(P.transpose(1, 2).contiguous(), dO)), KV)}
+        for name, (got, want, n) in ref.items():
+            num[name] = num.get(name, 0.0) + (heads(got, n) - want).pow(2).sum()
+            den[name] = den.get(name, 0.0) + want.pow(2).sum()
+        err["lse"] = max(err.get("lse", 0.0), float((lse[b].double() - torch.logsumexp(s, -1)).abs().max()))
+    for name in num:
+        err[name] = float((num[name] / den[name]).sqrt())
+    assert err["lse"] < 1e-3 and err["o"] < 1e-2, err
+    assert max(err["dq"], err["dk"], err["dv"]) < 2e-2, err
