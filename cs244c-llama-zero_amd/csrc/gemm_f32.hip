@@ -85,6 +85,7 @@ Plan make_plan(int64_t M, int64_t N, int64_t K) {
   static constexpr Tile kTiles[] = {{32, 128, 3.5, 0.85, 0.90}, {64, 32, 4.6, 0.70, 0.56}, {128, 32, 6.0, 2.30, 2.10}};
   static constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32, 48, 64};
   constexpr double kBytesPerUs = 5e6;
+  const int64_t cus = lz_num_cus();
   const double out = (double)M * N * sizeof(float) / kBytesPerUs;
   Plan best{64, 1, K};
   double least = INFINITY;
@@ -92,10 +93,10 @@ Plan make_plan(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = lz_cdiv(M, t.size) * lz_cdiv(N, t.size), deep = t.deep;
     for (const int want : kSplits) {
       // a split keeps a stage of its own, and 8 workgroups per CU need no more
-      if (want > 1 && (K < want * deep || tiles * want > 2048)) break;
+      if (want > 1 && (K < want * deep || tiles * want > 8 * cus)) break;
       const int64_t kper = want > 1 ? lz_cdiv(lz_cdiv(K, want), deep) * deep : K;
       const int64_t splits = want > 1 ? lz_cdiv(K, kper) : 1;
-      const double stages = (double)lz_cdiv(kper, deep), rounds = (double)lz_cdiv(tiles * splits, 256);
+      const double stages = (double)lz_cdiv(kper, deep), rounds = (double)lz_cdiv(tiles * splits, cus);
       double us = t.start + std::max(stages * t.chain, rounds * stages * t.busy) + out;
       if (splits > 1) us += 2.2 + 2.0 * splits * out;
       if (us < least) {
