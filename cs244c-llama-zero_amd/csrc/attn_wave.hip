@@ -19,10 +19,11 @@
 // the B operand of the second product as it stands: rows() forms tile . own^T
 // and cols() adds tile^T . P.
 // Measured against the kernels these calls had before (us, forward + dQ + dK/dV
-// device time, before -> after): heads 10/2 of 32, B 2, S 512: bf16 604 -> 33,
-// fp32 627 -> 83; heads 12/4 of 64, B 4, S 500, bool mask, bf16 6246 -> 106;
+// device time, before -> after): heads 10/2 of 32, B 2, S 512: bf16 604 -> 38,
+// fp32 627 -> 82; heads 12/4 of 64, B 4, S 500, bool mask, bf16 6246 -> 110;
 // forward of heads 16/8 of 128, B 1, S 777, bf16 59 (and a transposed copy of
-// V, 11) -> 19.
+// V, 11) -> 19.  The exact weights and the second pass that non-finite sums ask
+// for are 5 and 11 us of the two bf16 forward + backward figures.
 //
 //   PolF32: fp32 MFMAs (v_mfma_f32_32x32x2_f32) on fp32 tiles; fp32 and fp16
 //     operands.  Every value after the load is fp32.
@@ -848,8 +849,12 @@ __global__ void __launch_bounds__(64 * NW) attn_dkdv_wave_kernel(LzWaveArgs a) {
   sum_and_store<P, NW>(smem, kRegion, row_ptr_w<P>(a.dk, grow, a.lddk, (int64_t)g * HD), valid, a.scale, wave, lane);
 }
 
-// Waves per workgroup: eight (two per SIMD) while their LDS regions fit and
-// the registers of two waves per SIMD suffice, four otherwise.
+// Waves per workgroup: eight (two per SIMD) for heads of 32 and 16-bit heads of
+// 64, four where the LDS regions or the accumulators take more.  The general
+// bf16 dK/dV kernel for heads of 64 spills 34 of its registers at eight waves
+// and none at four, and is faster with eight: 12/4 heads, B 4, S 500, bool mask
+// 49.6 against 69.1 us.  The general dK/dV kernels for heads of 128 spill at four
+// (bf16 31, fp16 86, fp32 156 registers).
 template <class P>
 constexpr int waves_of() {
   return P::HD == 32 || (P::HD == 64 && P::k16) ? 8 : 4;
@@ -907,10 +912,11 @@ bool lz_attn_wave_ok(const LzWaveArgs& a, int dtype, int64_t hd, bool backward, 
 
 int lz_attn_wave_pass(const LzWaveArgs& a, int dtype, int64_t hd, LzWaveMode mode, LzWavePass pass, hipStream_t s) {
   const bool gen = mode == kWaveGeneral, split = mode == kWaveSplit;
+  // (heads of 32 are never rounded: no tile kernel takes them)
 #define LZ_WAVE(HD)                                                                              \
-  (dtype == LZ_BF16 ? (gen     ? launch<PolBF16<HD, true>, true>(a, pass, s)                 \
-                       : split ? launch<PolBF16<HD, true>, false>(a, pass, s)                \
-                               : launch<PolBF16<HD, false>, false>(a, pass, s))              \
+  (dtype == LZ_BF16 ? (gen                  ? launch<PolBF16<HD, true>, true>(a, pass, s)    \
+                       : split || HD == 32 ? launch<PolBF16<HD, true>, false>(a, pass, s)   \
+                                            : launch<PolBF16<HD, HD == 32>, false>(a, pass, s)) \
    : dtype == LZ_F16 ? (gen ? launch<PolF32<_Float16, HD>, true>(a, pass, s)                 \
                             : launch<PolF32<_Float16, HD>, false>(a, pass, s))               \
                      : (gen ? launch<PolF32<float, HD>, true>(a, pass, s)                    \

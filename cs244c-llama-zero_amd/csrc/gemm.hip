@@ -611,9 +611,6 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_dma_kernel(GemmArgs g) {
   gemm_dma_tile<F, WM, WN, AK, BK, DBK, NST, kEpiPlain>(g, SwigluOut{}, RopeIn{}, SwigluBwdIn{});
 }
 
-// 256x192 tiles (A K-major; B either layout; plain epilogue): for products
-// whose 256-wide tiles would leave CUs idle, e.g. N = 768 over 16384 rows,
-// where 4 column tiles of 192 make 256 workgroups and 3 of 256 only 192.
 // Weight gradients (both operands M/N-major) whose K, the token count, is not
 // a multiple of 64.
 template <typename F>
@@ -621,6 +618,9 @@ __global__ void __launch_bounds__(512) gemm_dma_tail_kernel(GemmArgs g) {
   gemm_dma_tile<F, 2, 4, false, false, 64, 2, kEpiPlain, 256, true>(g, SwigluOut{}, RopeIn{}, SwigluBwdIn{});
 }
 
+// 256x192 tiles (A K-major; B either layout; plain epilogue): for products
+// whose 256-wide tiles would leave CUs idle, e.g. N = 768 over 16384 rows,
+// where 4 column tiles of 192 make 256 workgroups and 3 of 256 only 192.
 template <typename F, bool BK>
 __global__ void __launch_bounds__(512) gemm_dma_n192_kernel(GemmArgs g) {
   gemm_dma_tile<F, 2, 4, true, BK, 64, 2, kEpiPlain, 192>(g, SwigluOut{}, RopeIn{}, SwigluBwdIn{});
@@ -994,10 +994,14 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, bool ak, bool bk) {
   // The small tiles where they are clearly faster than that plan (the
   // register-staged kernel's time taken as 1.8 times the direct-to-LDS
   // one's): few rows or columns, a short grid, a K that is not a multiple of 64.
-  // Over the products the costs were fitted to, this takes 0.48 of the
-  // time (geometric mean) and is at most 6 % slower on one (768x2048x8192
-  // dy^T.x); e.g. 333x768x768 17.5 -> 7.1 us, 768x768x2000 dy^T.x 57 -> 13.5,
-  // 777x4096x2048 41 -> 23.
+  // Over 660 of the products the costs were fitted to, all products take 0.50
+  // of the time they took without them (geometric mean) and none is more than
+  // 5 % slower; e.g. 333x768x768 17.5 -> 7.1 us, 768x768x2000 dy^T.x 57 -> 13.5,
+  // 777x4096x2048 41 -> 23.  The fit ends at K 8192 and the slabs' cost grows
+  // wrong beyond it: of the 91 products of K 12296 .. 32000 that would take small
+  // tiles without the bound on K most gain (333x320x16384 36 -> 20) but long
+  // weight gradients of wider outputs lose (256x688x32768 dy^T.x 47 -> 60,
+  // 1376x256x20000 44 -> 53).
   if ((ak || !bk) && min_splits == 1 && K <= 12288) {
     const double old = p.cfg >= 5 ? plan_us(p.cfg, p.splits, M, N, K, bk, ak) : 1.8 * plan_us(5, p.splits, M, N, K, bk, ak);
     double best = 0.8 * old;
