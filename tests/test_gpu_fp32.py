@@ -79,6 +79,28 @@ def test_gemm_f32_tiles_and_tails_vs_float64(ak, bk, M, N, K):
     assert _rel(out, ref) <= 2.0 ** -24 * (8 + (K / 64) ** 0.5)
 
 
+@pytest.mark.parametrize("ak,bk", [(True, True), (True, False), (False, True), (False, False)])
+@pytest.mark.parametrize("aoff,boff", [(1, 0), (0, 2), (3, 1)])
+@pytest.mark.parametrize("M,N,K", [(3, 2, 3), (70, 131, 129), (641, 2049, 95), (260, 100, 4099)])
+def test_gemm_f32_rows_at_any_float(ak, bk, aoff, boff, M, N, K):
+    """Operands whose rows start at any float, one or both, with short ends of
+    one to three floats and NaN around them: nothing outside an operand reaches
+    a result.  Bound as test_gemm_f32_tiles_and_tails_vs_float64."""
+    g = torch.Generator(device=DEV).manual_seed(M + N + K + aoff + boff)
+
+    def operand(t, kmajor, off):
+        t = t if kmajor else t.t()
+        buf = torch.full((t.shape[0] + 1, t.shape[1] + 5), float("nan"), device=DEV)
+        view = buf[: t.shape[0], off : off + t.shape[1]]
+        view.copy_(t)
+        return view
+
+    a, b = torch.randn(M, K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    out = ops.gemm(operand(a, ak, aoff), operand(b, bk, boff), ak, bk)
+    ref = a.double() @ b.double().t()
+    assert _rel(out, ref) <= 2.0 ** -24 * (8 + (K / 64) ** 0.5)
+
+
 def test_gemm_f32_split_plan():
     """Few output tiles with a long K (a language-model head's input
     gradient: 512 tokens x 256 features over a 32000 vocabulary) are split
